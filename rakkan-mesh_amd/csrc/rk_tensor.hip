@@ -3,18 +3,32 @@
 // quantize / scale that produce and consume the i8 form.
 //
 // f32 (tensor.go:318-327): c_ij = Canonical(acc), acc += float32(a_ip·b_pj)
-// for p = 0..k-1 from +0 — a sequential sum per output, so each output is
-// one lane's chain of multiplies and adds on the vector ALUs (a matrix
-// core's reduction tree would round differently). A workgroup stages
-// 64-position slices of its 32 rows of a and 32 columns of b in LDS (b as
-// columns, so both read four positions per 16-byte load) and each thread
-// runs four chains (2 rows x 2 columns).
+// for p = 0..k-1 from +0, a sequential sum per output. The products of a
+// 16x16 tile at one position are an outer product: v_mfma_f32_16x16x1 with a
+// zero accumulator gives four positions' rounded products at once (a K = 1
+// result is one product plus +0: only the sign of a zero is lost, and a sum
+// that starts at +0 never is -0, so adding either zero leaves it), and the
+// vector ALU does the adds alone, in order. What bounds it: an add and a
+// product a position, 16 adds (2.3 cycles each) and one matrix instruction
+// (34 cycles) per 1024 products, which measured one after the other on
+// MI355X, not together: 24.5 us of a 1024 x 784 x 1024 product. It takes 38
+// us (75 us with two outputs a side a thread from LDS, products on the vector
+// ALU: operand reads, tests and the loads' latency).
 //
 // i8 (tensor.go:328-335): c_ij = Σ int32(a_ip)·int32(b_pj) with Go's int32
-// wraparound. Integer sums are exact in any order, so the block sums run on
-// int8 MFMA (v_mfma_i32_16x16x32_i8, accumulator chained); the accumulator
+// wraparound. Integer sums are exact in any order, so the sums run on int8
+// MFMA (v_mfma_i32_16x16x64_i8, accumulator chained); the accumulator
 // restarts every 65536 positions (|partial| <= 2^30, no overflow inside the
-// matrix core) and the partials are added with wrapping integer adds.
+// matrix core) and the partials are added with wrapping integer adds. What
+// bounds it: LDS reads and the staging of slices (16 bytes a lane and row;
+// b[k][n] turned in registers, 4x4 bytes at a time, so that both operands
+// read 16 positions of a row or column as one LDS load). 2048^3: 25.5 us,
+// 337 TMAC/s (21 us with b[n][k]), against 226 us with byte loads, 8-byte
+// LDS reads and no load in flight during the sums.
+//
+// Both load the next slice while this one is summed (two LDS slices, one
+// barrier a slice). A slice that is whole takes no tests: a test around a
+// load makes the compiler wait for it there.
 #include <algorithm>
 #include <mutex>
 
@@ -27,172 +41,339 @@ namespace rk {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int rk_i2 __attribute__((ext_vector_type(2)));
 
-// ---- f32 ----
-constexpr int kTfTile = 32;    // outputs per side of a workgroup
-constexpr int kTfChunk = 64;   // positions per staged slice
-constexpr int kTfPitch = kTfChunk + 4;
-
-__global__ __launch_bounds__(256) void tensor_mm_f32_kernel(const float *a, const float *b, float *c, int64_t m,
-                                                            int64_t k, int64_t n, int transposed) {
-    __shared__ __align__(16) float sa[kTfTile][kTfPitch];  // rows of a
-    __shared__ __align__(16) float sb[kTfTile][kTfPitch];  // columns of b
-    const int tid = threadIdx.x;
-    const int64_t i0 = (int64_t)blockIdx.y * kTfTile, j0 = (int64_t)blockIdx.x * kTfTile;
-    // thread -> rows i0 + ti, i0 + ti + 16 and columns j0 + tj, j0 + tj + 16
-    const int ti = tid >> 4, tj = tid & 15;
-    float acc[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
-    for (int64_t p0 = 0; p0 < k; p0 += kTfChunk) {
-        const int np = (int)min((int64_t)kTfChunk, k - p0);
-        // stage: 32 x 64 of each (zeros past k are never summed)
-        for (int e = tid; e < kTfTile * kTfChunk; e += 256) {
-            const int r = e / kTfChunk, p = e % kTfChunk;
-            const int64_t gi = min(i0 + r, m - 1), gp = min(p0 + p, k - 1);
-            sa[r][p] = a[gi * k + gp];
-        }
-        if (transposed) {  // b[n][k]: column j of the product is row j
-            for (int e = tid; e < kTfTile * kTfChunk; e += 256) {
-                const int r = e / kTfChunk, p = e % kTfChunk;
-                const int64_t gj = min(j0 + r, n - 1), gp = min(p0 + p, k - 1);
-                sb[r][p] = b[gj * k + gp];
-            }
-        } else {  // b[k][n]: read along n, store as columns
-            for (int e = tid; e < kTfTile * kTfChunk; e += 256) {
-                const int p = e / kTfTile, r = e % kTfTile;
-                const int64_t gj = min(j0 + r, n - 1), gp = min(p0 + p, k - 1);
-                sb[r][p] = b[gp * n + gj];
-            }
-        }
-        __syncthreads();
-        const float *ra0 = sa[ti], *ra1 = sa[ti + 16], *rb0 = sb[tj], *rb1 = sb[tj + 16];
-        int p = 0;
-        for (; p + 4 <= np; p += 4) {
-            const float4 x0 = *reinterpret_cast<const float4 *>(ra0 + p);
-            const float4 x1 = *reinterpret_cast<const float4 *>(ra1 + p);
-            const float4 y0 = *reinterpret_cast<const float4 *>(rb0 + p);
-            const float4 y1 = *reinterpret_cast<const float4 *>(rb1 + p);
-            const float xa[2][4] = {{x0.x, x0.y, x0.z, x0.w}, {x1.x, x1.y, x1.z, x1.w}};
-            const float yb[2][4] = {{y0.x, y0.y, y0.z, y0.w}, {y1.x, y1.y, y1.z, y1.w}};
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-#pragma unroll
-                for (int r = 0; r < 2; r++)
-#pragma unroll
-                    for (int s = 0; s < 2; s++) acc[r][s] += xa[r][q] * yb[s][q];
-        }
-        for (; p < np; p++)
-#pragma unroll
-            for (int r = 0; r < 2; r++)
-#pragma unroll
-                for (int s = 0; s < 2; s++) acc[r][s] += sa[ti + 16 * r][p] * sb[tj + 16 * s][p];
-        __syncthreads();
-    }
-#pragma unroll
-    for (int r = 0; r < 2; r++)
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const int64_t i = i0 + ti + 16 * r, j = j0 + tj + 16 * s;
-            if (i < m && j < n) c[i * n + j] = canonical(acc[r][s]);
-        }
+// Tile order: workgroup ids go round the 8 XCDs, so id mod 8 picks a
+// contiguous run of tiles (along n first): an XCD's workgroups then share
+// rows of a and columns of b in its own L2. -1: past the last tile.
+__device__ __forceinline__ int64_t xcd_tile(int64_t tiles) {
+    const int64_t per = (tiles + 7) >> 3, t = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    return (blockIdx.x >> 3) < per && t < tiles ? t : -1;
 }
 
-// ---- i8 ----
-constexpr int kTiTile = 64;    // outputs per side of a workgroup
-constexpr int kTiChunk = 256;  // positions per staged slice
-constexpr int kTiPitch = kTiChunk + 8;  // bytes: 16 rows at one offset in distinct banks
-constexpr int64_t kTiRestart = 65536;   // positions per matrix-core accumulation
+// ---- f32 ----
+constexpr int kTfTile = 32;    // outputs per side of a workgroup: 16 per side a wave
+constexpr int kTfChunk = 64;   // positions per staged slice
+constexpr int kTfPitch = kTfChunk + 4;
+constexpr int kTfLoads = kTfTile * kTfChunk / 4 / 256;  // 16-byte loads a thread and operand
 
-__global__ __launch_bounds__(256) void tensor_mm_i8_kernel(const int8_t *a, const int8_t *b, int32_t *c, int64_t m,
-                                                           int64_t k, int64_t n, int transposed) {
-    __shared__ __align__(16) int8_t sa[kTiTile][kTiPitch];  // rows of a
-    __shared__ __align__(16) int8_t sb[kTiTile][kTiPitch];  // columns of b
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+// Four floats from `at` of an array of `total` (>= 4), zeros past the first
+// `valid`: near the array's end the load moves back into it and what
+// precedes `at` is dropped.
+__device__ __forceinline__ float4 tf_edge4(const float *x, int64_t at, int64_t total, int64_t valid) {
+    const int64_t q = min(at, total - 4);
+    const int o = (int)min(at - q, (int64_t)4);
+    float4 v;
+    __builtin_memcpy(&v, x + q, 16);
+    if (o & 1) v = make_float4(v.y, v.z, v.w, 0.0f);
+    if (o & 2) v = make_float4(v.z, v.w, 0.0f, 0.0f);
+    if (o & 4) v.x = 0.0f;
+    return make_float4(valid > 0 ? v.x : 0.0f, valid > 1 ? v.y : 0.0f, valid > 2 ? v.z : 0.0f, valid > 3 ? v.w : 0.0f);
+}
+
+template <bool TRANS>
+__global__ __launch_bounds__(256, 4) void tensor_mm_f32_kernel(const float *a, const float *b, float *c, int64_t m,
+                                                               int64_t k, int64_t n) {
+    __shared__ __align__(16) float sa[2][kTfTile][kTfPitch];  // rows of a
+    __shared__ __align__(16) float sb[2][kTfTile][kTfPitch];  // columns of b
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lq = lane >> 4, ln = lane & 15;
-    const int wr = wave & 1, wc = wave >> 1;  // the wave's 32 x 32 quarter
-    const int64_t i0 = (int64_t)blockIdx.y * kTiTile, j0 = (int64_t)blockIdx.x * kTiTile;
-    v4i d[2][2];
-    int32_t tot[2][2][4];
+    const int64_t tn = (n + kTfTile - 1) / kTfTile;
+    const int64_t t = xcd_tile((m + kTfTile - 1) / kTfTile * tn);
+    if (t < 0) return;  // uniform
+    const int64_t i0 = t / tn * kTfTile, j0 = t % tn * kTfTile;
+    // a slice's loads; rows past m and columns past n repeat others (never
+    // stored); positions past k are zeros, whose products add +0. Whole
+    // slices (all but the last; b[k][n]'s last columns read on into the next
+    // row, so there whole slices end before the last row) take no tests.
+    float4 va[kTfLoads], vb[kTfLoads];
+    const float *ra[kTfLoads], *rb[kTfLoads];
 #pragma unroll
-    for (int r = 0; r < 2; r++)
+    for (int e = 0; e < kTfLoads; e++) {
+        const int u = tid + 256 * e, r = u / (kTfChunk / 4), p = 4 * (u % (kTfChunk / 4));
+        ra[e] = a + min(i0 + r, m - 1) * k + p;
+        const int64_t j = j0 + 4 * (u % (kTfTile / 4));
+        rb[e] = TRANS ? b + min(j0 + r, n - 1) * k + p : b + (u / (kTfTile / 4)) * n + (j < n ? j : 0);
+    }
+    const int64_t whole = TRANS || n % 4 == 0 ? k : k - 4;
+    auto load = [&](int64_t p0) {
+        if (p0 + kTfChunk <= whole) {  // uniform
 #pragma unroll
-        for (int s = 0; s < 2; s++) {
-            d[r][s] = v4i{0, 0, 0, 0};
-#pragma unroll
-            for (int e = 0; e < 4; e++) tot[r][s][e] = 0;
-        }
-    for (int64_t p0 = 0; p0 < k; p0 += kTiChunk) {
-        // stage 64 x 256 of each; positions past k are zeros (they add 0)
-        for (int e = tid; e < kTiTile * (kTiChunk / 4); e += 256) {
-            const int r = e / (kTiChunk / 4), p = 4 * (e % (kTiChunk / 4));
-            const int64_t gi = min(i0 + r, m - 1);
-            uint32_t w = 0;
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                if (p0 + p + q < k) w |= (uint32_t)(uint8_t)a[gi * k + p0 + p + q] << (8 * q);
-            *reinterpret_cast<uint32_t *>(&sa[r][p]) = w;
-        }
-        if (transposed) {
-            for (int e = tid; e < kTiTile * (kTiChunk / 4); e += 256) {
-                const int r = e / (kTiChunk / 4), p = 4 * (e % (kTiChunk / 4));
-                const int64_t gj = min(j0 + r, n - 1);
-                uint32_t w = 0;
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-                    if (p0 + p + q < k) w |= (uint32_t)(uint8_t)b[gj * k + p0 + p + q] << (8 * q);
-                *reinterpret_cast<uint32_t *>(&sb[r][p]) = w;
+            for (int e = 0; e < kTfLoads; e++) {
+                __builtin_memcpy(&va[e], ra[e] + p0, 16);
+                __builtin_memcpy(&vb[e], rb[e] + (TRANS ? p0 : p0 * n), 16);
             }
         } else {
-            for (int e = tid; e < kTiTile * (kTiChunk / 4); e += 256) {
-                const int r = e % kTiTile, p = 4 * (e / kTiTile);
-                const int64_t gj = min(j0 + r, n - 1);
-                uint32_t w = 0;
 #pragma unroll
-                for (int q = 0; q < 4; q++)
-                    if (p0 + p + q < k) w |= (uint32_t)(uint8_t)b[(p0 + p + q) * n + gj] << (8 * q);
-                *reinterpret_cast<uint32_t *>(&sb[r][p]) = w;
+            for (int e = 0; e < kTfLoads; e++) {
+                const int u = tid + 256 * e, p = 4 * (u % (kTfChunk / 4));
+                va[e] = tf_edge4(a, ra[e] - a + p0, m * k, k - p0 - p);
+                if constexpr (TRANS)
+                    vb[e] = tf_edge4(b, rb[e] - b + p0, n * k, k - p0 - p);
+                else
+                    vb[e] = tf_edge4(b, rb[e] - b + p0 * n, n * k, p0 + u / (kTfTile / 4) < k ? 4 : 0);
+            }
+        }
+    };
+    const int ar = 16 * (wave >> 1) + ln, bc = 16 * (wave & 1) + ln;  // the wave's row of a, column of b
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    load(0);
+    int s = 0;
+    for (int64_t p0 = 0; p0 < k; p0 += kTfChunk, s ^= 1) {
+#pragma unroll
+        for (int e = 0; e < kTfLoads; e++) {
+            const int u = tid + 256 * e, r = u / (kTfChunk / 4), p = 4 * (u % (kTfChunk / 4));
+            *reinterpret_cast<float4 *>(&sa[s][r][p]) = va[e];
+            if constexpr (TRANS) {
+                *reinterpret_cast<float4 *>(&sb[s][r][p]) = vb[e];
+            } else {
+                const int q = u / (kTfTile / 4), j = 4 * (u % (kTfTile / 4));
+                sb[s][j][q] = vb[e].x;
+                sb[s][j + 1][q] = vb[e].y;
+                sb[s][j + 2][q] = vb[e].z;
+                sb[s][j + 3][q] = vb[e].w;
             }
         }
         __syncthreads();
+        if (p0 + kTfChunk < k) load(p0 + kTfChunk);
+#pragma unroll 4
+        for (int p = 0; p < kTfChunk; p += 4) {
+            // block q of the matrix core's four takes position p + q: its
+            // four results are elements 4q .. 4q + 3
+            const v16f z = {};
+            const v16f d =
+                __builtin_amdgcn_mfma_f32_16x16x1f32(sa[s][ar][p + lq], sb[s][bc][p + lq], z, 0, 0, 0);
 #pragma unroll
-        for (int ks = 0; ks < kTiChunk / 32; ks++) {
-            long fa[2], fb[2];
+            for (int q = 0; q < 4; q++)
 #pragma unroll
-            for (int r = 0; r < 2; r++)
-                fa[r] = *reinterpret_cast<const long *>(&sa[32 * wr + 16 * r + ln][32 * ks + 8 * lq]);
-#pragma unroll
-            for (int s = 0; s < 2; s++)
-                fb[s] = *reinterpret_cast<const long *>(&sb[32 * wc + 16 * s + ln][32 * ks + 8 * lq]);
-#pragma unroll
-            for (int r = 0; r < 2; r++)
-#pragma unroll
-                for (int s = 0; s < 2; s++) d[r][s] = __builtin_amdgcn_mfma_i32_16x16x32_i8(fa[r], fb[s], d[r][s], 0, 0, 0);
-        }
-        __syncthreads();
-        if ((p0 + kTiChunk) % kTiRestart == 0 || p0 + kTiChunk >= k) {
-            // fold the matrix core's partial into the wrapping total
-#pragma unroll
-            for (int r = 0; r < 2; r++)
-#pragma unroll
-                for (int s = 0; s < 2; s++) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        tot[r][s][e] = (int32_t)((uint32_t)tot[r][s][e] + (uint32_t)d[r][s][e]);
-                    d[r][s] = v4i{0, 0, 0, 0};
-                }
+                for (int e = 0; e < 4; e++) acc[e] += d[4 * q + e];
         }
     }
     // the 16x16 result layout: lane holds column ln, rows 4·lq + e
+    const int64_t j = j0 + 16 * (wave & 1) + ln;
 #pragma unroll
-    for (int r = 0; r < 2; r++)
+    for (int e = 0; e < 4; e++) {
+        const int64_t i = i0 + 16 * (wave >> 1) + 4 * lq + e;
+        if (i < m && j < n) c[i * n + j] = canonical(acc[e]);
+    }
+}
+
+// ---- i8 ----
+constexpr int64_t kTiRestart = 65536;   // positions per matrix-core accumulation
+
+// 16 bytes from `at` of an array of `total` (>= 16), zeros past the first
+// `valid` (any alignment); near the array's end as tf_edge4.
+__device__ __forceinline__ v4i ti_edge16(const int8_t *x, int64_t at, int64_t total, int64_t valid) {
+    const int64_t q = min(at, total - 16);
+    const int o = (int)min(at - q, (int64_t)16), keep = (int)max(min(valid, (int64_t)16), (int64_t)0);
+    unsigned __int128 w;
+    __builtin_memcpy(&w, x + q, 16);
+    w = o < 16 ? w >> (8 * o) : 0;
+    w = keep == 16 ? w : w & (((unsigned __int128)1 << (8 * keep)) - 1);
+    v4i v;
+    __builtin_memcpy(&v, &w, 16);
+    return v;
+}
+
+// Four bytes from `at`, zeros unless `valid`, likewise.
+__device__ __forceinline__ int ti_edge4(const int8_t *x, int64_t at, int64_t total, bool valid) {
+    const int64_t q = min(at, total - 4);
+    const int o = (int)min(at - q, (int64_t)4);
+    uint32_t v;
+    __builtin_memcpy(&v, x + q, 4);
+    return valid && o < 4 ? (int)(v >> (8 * o)) : 0;
+}
+
+// A workgroup of four waves forms TM x TN outputs from slices of KC
+// positions: WM x WN waves side by side, WK waves sharing each part's
+// positions (their integer partials added at the end).
+template <int TM, int TN, int KC, int WM, int WN, int WK, bool TRANS>
+__global__ __launch_bounds__(256) void tensor_mm_i8_kernel(const int8_t *a, const int8_t *b, int32_t *c, int64_t m,
+                                                           int64_t k, int64_t n) {
+    constexpr int PITCH = KC + 16;    // bytes: 16 rows at one offset in distinct banks
+    constexpr int NA = TM * KC / 16 / 256, NB = TN * KC / 16 / 256;  // 16-byte loads a thread
+    constexpr int RM = TM / WM / 16, RN = TN / WN / 16;              // 16x16 results a wave
+    // b[k][n]: a thread takes 8 positions of 4 columns and turns them; its
+    // low lane bits spread over columns and positions so that the turned
+    // columns' stores fall in distinct banks
+    constexpr int CG = TN / 4, KG = 256 / CG, NU = KC / 8 / KG;
+    static_assert(WM * WN * WK == 4 && NA >= 1 && NB >= 1 && NU >= 1 && CG >= 8, "four waves, whole loads");
+    extern __shared__ __align__(16) int8_t ti_lds[];
+    int8_t *sa = ti_lds, *sb = ti_lds + 2 * TM * PITCH;  // rows of a, columns of b, two slices each
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lq = lane >> 4, ln = lane & 15;
+    const int wk = wave % WK, wn = wave / WK % WN, wm = wave / WK / WN;
+    const int64_t tn = (n + TN - 1) / TN;
+    const int64_t t = xcd_tile((m + TM - 1) / TM * tn);
+    if (t < 0) return;  // uniform
+    const int64_t i0 = t / tn * TM, j0 = t % tn * TN;
+    const int cg = (tid & 3) | (tid >> 5) % (CG / 4) * 4, kg = (tid >> 2 & 7) | (tid >> 5) / (CG / 4) * 8;
+    const int64_t jc = j0 + 4 * cg < n ? j0 + 4 * cg : 0;
+    // as in the f32 kernel: rows and columns past the end repeat others,
+    // positions past k are zeros, whole slices take no tests
+    v4i va[NA], vb[NB];
+    int vc[NU][8];
+    const int8_t *ra[NA], *rb[NB];
 #pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const int64_t j = j0 + 32 * wc + 16 * s + ln;
+    for (int e = 0; e < NA; e++) {
+        const int u = tid + 256 * e;
+        ra[e] = a + min(i0 + u / (KC / 16), m - 1) * k + 16 * (u % (KC / 16));
+    }
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int64_t i = i0 + 32 * wr + 16 * r + 4 * lq + e;
-                if (i < m && j < n) c[i * n + j] = tot[r][s][e];
+    for (int e = 0; e < NB; e++) {
+        const int u = tid + 256 * e;
+        rb[e] = b + min(j0 + u / (KC / 16), n - 1) * k + 16 * (u % (KC / 16));
+    }
+    const int64_t whole = TRANS || n % 4 == 0 ? k : k - 4;
+    auto load = [&](int64_t p0) {
+        if (p0 + KC <= whole) {  // uniform
+#pragma unroll
+            for (int e = 0; e < NA; e++) __builtin_memcpy(&va[e], ra[e] + p0, 16);
+            if constexpr (TRANS) {
+#pragma unroll
+                for (int e = 0; e < NB; e++) __builtin_memcpy(&vb[e], rb[e] + p0, 16);
+            } else {
+#pragma unroll
+                for (int u = 0; u < NU; u++) {
+                    const int8_t *q = b + (p0 + 8 * (kg + KG * u)) * n + jc;
+#pragma unroll
+                    for (int e = 0; e < 8; e++, q += n) __builtin_memcpy(&vc[u][e], q, 4);
+                }
+            }
+        } else {
+            const int p = 16 * (tid % (KC / 16));  // the same for each e (256 threads are whole rows)
+#pragma unroll
+            for (int e = 0; e < NA; e++) va[e] = ti_edge16(a, ra[e] - a + p0, m * k, k - p0 - p);
+            if constexpr (TRANS) {
+#pragma unroll
+                for (int e = 0; e < NB; e++) vb[e] = ti_edge16(b, rb[e] - b + p0, n * k, k - p0 - p);
+            } else {
+#pragma unroll
+                for (int u = 0; u < NU; u++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const int64_t q = p0 + 8 * (kg + KG * u) + e;
+                        vc[u][e] = ti_edge4(b, q * n + jc, n * k, q < k);
+                    }
             }
         }
+    };
+    auto store = [&](int s) {
+#pragma unroll
+        for (int e = 0; e < NA; e++) {
+            const int u = tid + 256 * e;
+            *reinterpret_cast<v4i *>(sa + (s * TM + u / (KC / 16)) * PITCH + 16 * (u % (KC / 16))) = va[e];
+        }
+        if constexpr (TRANS) {
+#pragma unroll
+            for (int e = 0; e < NB; e++) {
+                const int u = tid + 256 * e;
+                *reinterpret_cast<v4i *>(sb + (s * TN + u / (KC / 16)) * PITCH + 16 * (u % (KC / 16))) = vb[e];
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < NU; u++) {
+                rk_i2 col[4];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {  // a 4x4 turn of bytes
+                    const int *x = vc[u] + 4 * h;
+                    const uint32_t l01 = __builtin_amdgcn_perm(x[1], x[0], 0x05010400);
+                    const uint32_t h01 = __builtin_amdgcn_perm(x[1], x[0], 0x07030602);
+                    const uint32_t l23 = __builtin_amdgcn_perm(x[3], x[2], 0x05010400);
+                    const uint32_t h23 = __builtin_amdgcn_perm(x[3], x[2], 0x07030602);
+                    col[0][h] = (int)__builtin_amdgcn_perm(l23, l01, 0x05040100);
+                    col[1][h] = (int)__builtin_amdgcn_perm(l23, l01, 0x07060302);
+                    col[2][h] = (int)__builtin_amdgcn_perm(h23, h01, 0x05040100);
+                    col[3][h] = (int)__builtin_amdgcn_perm(h23, h01, 0x07060302);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    *reinterpret_cast<rk_i2 *>(sb + (s * TN + 4 * cg + e) * PITCH + 8 * (kg + KG * u)) = col[e];
+            }
+        }
+    };
+    for (int64_t k0 = 0; k0 < k; k0 += kTiRestart) {  // uniform; one pass up to 65536 positions
+        const int64_t k1 = min(k, k0 + kTiRestart);
+        v4i d[RM][RN];
+#pragma unroll
+        for (int r = 0; r < RM; r++)
+#pragma unroll
+            for (int q = 0; q < RN; q++) d[r][q] = v4i{0, 0, 0, 0};
+        load(k0);
+        int s = 0;
+        for (int64_t p0 = k0; p0 < k1; p0 += KC, s ^= 1) {
+            store(s);
+            __syncthreads();
+            if (p0 + KC < k1) load(p0 + KC);
+#pragma unroll
+            for (int ks = 0; ks < KC / WK; ks += 64) {
+                const int at = wk * (KC / WK) + ks + 16 * lq;
+                v4i fa[RM], fb[RN];
+#pragma unroll
+                for (int r = 0; r < RM; r++)
+                    fa[r] = *reinterpret_cast<const v4i *>(sa + (s * TM + (wm * RM + r) * 16 + ln) * PITCH + at);
+#pragma unroll
+                for (int q = 0; q < RN; q++)
+                    fb[q] = *reinterpret_cast<const v4i *>(sb + (s * TN + (wn * RN + q) * 16 + ln) * PITCH + at);
+#pragma unroll
+                for (int r = 0; r < RM; r++)
+#pragma unroll
+                    for (int q = 0; q < RN; q++)
+                        d[r][q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[r], fb[q], d[r][q], 0, 0, 0);
+            }
+        }
+        __syncthreads();  // the slices are read before they are written again
+        if constexpr (WK > 1) {
+            // the waves' partials through LDS, wrapping adds
+            int32_t *red = reinterpret_cast<int32_t *>(ti_lds);  // [WK][TM][TN]: within the slices
+#pragma unroll
+            for (int r = 0; r < RM; r++)
+#pragma unroll
+                for (int q = 0; q < RN; q++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        red[(wk * TM + (wm * RM + r) * 16 + 4 * lq + e) * TN + (wn * RN + q) * 16 + ln] = d[r][q][e];
+            __syncthreads();
+            for (int o = tid; o < TM * TN; o += 256) {
+                uint32_t v = 0;
+#pragma unroll
+                for (int w = 0; w < WK; w++) v += (uint32_t)red[w * TM * TN + o];
+                const int64_t i = i0 + o / TN, j = j0 + o % TN;
+                if (i < m && j < n) c[i * n + j] = (int32_t)(k0 ? (uint32_t)c[i * n + j] + v : v);
+            }
+            __syncthreads();
+        } else {
+            // the 16x16 result layout: lane holds column ln, rows 4·lq + e
+#pragma unroll
+            for (int r = 0; r < RM; r++)
+#pragma unroll
+                for (int q = 0; q < RN; q++) {
+                    const int64_t j = j0 + (wn * RN + q) * 16 + ln;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int64_t i = i0 + (wm * RM + r) * 16 + 4 * lq + e;
+                        const uint32_t v = (uint32_t)d[r][q][e];
+                        if (i < m && j < n) c[i * n + j] = (int32_t)(k0 ? (uint32_t)c[i * n + j] + v : v);
+                    }
+                }
+        }
+    }
+}
+
+// Operands smaller than a load (fewer than 4 floats or 16 bytes, so k < 16):
+// a thread an output.
+template <typename T, typename R>
+__global__ __launch_bounds__(256) void tensor_mm_small_kernel(const T *a, const T *b, R *c, int64_t m, int64_t k,
+                                                              int64_t n, int transposed) {
+    for (int64_t o = (int64_t)blockIdx.x * 256 + threadIdx.x; o < m * n; o += (int64_t)gridDim.x * 256) {
+        const int64_t i = o / n, j = o % n;
+        R v = 0;
+        for (int64_t p = 0; p < k; p++) v += (R)a[i * k + p] * (R)b[transposed ? j * k + p : p * n + j];
+        if constexpr (sizeof(T) == 4) v = canonical(v);
+        c[o] = v;
+    }
 }
 
 // ---- elementwise ----
@@ -216,25 +397,75 @@ __global__ void tensor_scale_kernel(const void *a, int i32, float *out, int64_t 
 
 }  // namespace
 
+static unsigned elem_grid(int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256, 65536); }
+
+static int64_t tiles_of(int64_t m, int64_t n, int tm, int tn) { return ((m + tm - 1) / tm) * ((n + tn - 1) / tn); }
+
+// One workgroup a tile, the count padded to whole rounds of the 8 XCDs
+// (xcd_tile). 2^31 tiles are 2^41 outputs: more than the memory.
+static dim3 tile_grid(int64_t m, int64_t n, int tm, int tn) { return dim3((unsigned)((tiles_of(m, n, tm, tn) + 7) / 8 * 8)); }
+
+template <int TM, int TN, int KC, int WM, int WN, int WK, bool TRANS>
+static void launch_tensor_i8_t(const int8_t *a, const int8_t *b, int32_t *c, int64_t m, int64_t k, int64_t n,
+                               hipStream_t s) {
+    constexpr int lds = 2 * (TM + TN) * (KC + 16);
+    static std::once_flag once;
+    std::call_once(once, [] {
+        (void)hipFuncSetAttribute((const void *)tensor_mm_i8_kernel<TM, TN, KC, WM, WN, WK, TRANS>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    });
+    RK_LAUNCH((tensor_mm_i8_kernel<TM, TN, KC, WM, WN, WK, TRANS>), tile_grid(m, n, TM, TN), dim3(256), lds, s, a, b, c,
+              m, k, n);
+}
+
+template <bool TRANS>
+static void launch_tensor_i8(const int8_t *a, const int8_t *b, int32_t *c, int64_t m, int64_t k, int64_t n,
+                             hipStream_t s) {
+    // The largest tile that still gives the chip's 256 CUs a workgroup or two
+    // each; below 128 tiles of 64 the 32 x 32 one, whose four waves share a
+    // slice of 512 positions, unless k would leave most of that slice empty.
+    // Measured (us, k x n operand b): 2048^3 25.5 / 33.5 at 64 / 105 at 32;
+    // 1024^3 9.7 / 7.4 / 16.4; 256 x 2048 x 256 15.2 / 11.1 / 6.4;
+    // 118 x 45 x 279 6.3 / 4.9 / 6.2.
+    if (tiles_of(m, n, 128, 64) >= 256)
+        launch_tensor_i8_t<128, 64, 128, 2, 2, 1, TRANS>(a, b, c, m, k, n, s);
+    else if (tiles_of(m, n, 64, 64) >= 128 || k < 512)
+        launch_tensor_i8_t<64, 64, 128, 2, 2, 1, TRANS>(a, b, c, m, k, n, s);
+    else
+        launch_tensor_i8_t<32, 32, 512, 1, 1, 4, TRANS>(a, b, c, m, k, n, s);
+}
+
 int enqueue_tensor_matmul(rk_device *d, int32_t dtype, int32_t transposed, int64_t m, int64_t k, int64_t n,
                           const void *a, const void *b, void *c, hipStream_t s) {
+    const int64_t least = std::min(m, n) * k;  // the smaller operand's elements
     if (dtype == RK_TENSOR_F32) {
-        const dim3 grid((unsigned)((n + kTfTile - 1) / kTfTile), (unsigned)((m + kTfTile - 1) / kTfTile));
         ProfScope p(d, s, "tensor_matmul_f32");
-        RK_LAUNCH(tensor_mm_f32_kernel, grid, dim3(256), 0, s, static_cast<const float *>(a),
-                  static_cast<const float *>(b), static_cast<float *>(c), m, k, n, transposed ? 1 : 0);
+        const float *fa = static_cast<const float *>(a), *fb = static_cast<const float *>(b);
+        float *fc = static_cast<float *>(c);
+        const dim3 grid = tile_grid(m, n, kTfTile, kTfTile);
+        if (least < 4)
+            RK_LAUNCH((tensor_mm_small_kernel<float, float>), dim3(elem_grid(m * n)), dim3(256), 0, s, fa, fb, fc, m, k,
+                      n, transposed);
+        else if (transposed)
+            RK_LAUNCH(tensor_mm_f32_kernel<true>, grid, dim3(256), 0, s, fa, fb, fc, m, k, n);
+        else
+            RK_LAUNCH(tensor_mm_f32_kernel<false>, grid, dim3(256), 0, s, fa, fb, fc, m, k, n);
     } else {
-        const dim3 grid((unsigned)((n + kTiTile - 1) / kTiTile), (unsigned)((m + kTiTile - 1) / kTiTile));
         ProfScope p(d, s, "tensor_matmul_i8");
-        RK_LAUNCH(tensor_mm_i8_kernel, grid, dim3(256), 0, s, static_cast<const int8_t *>(a),
-                  static_cast<const int8_t *>(b), static_cast<int32_t *>(c), m, k, n, transposed ? 1 : 0);
+        const int8_t *ia = static_cast<const int8_t *>(a), *ib = static_cast<const int8_t *>(b);
+        int32_t *ic = static_cast<int32_t *>(c);
+        if (least < 16)
+            RK_LAUNCH((tensor_mm_small_kernel<int8_t, int32_t>), dim3(elem_grid(m * n)), dim3(256), 0, s, ia, ib, ic, m,
+                      k, n, transposed);
+        else if (transposed)
+            launch_tensor_i8<true>(ia, ib, ic, m, k, n, s);
+        else
+            launch_tensor_i8<false>(ia, ib, ic, m, k, n, s);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(d, e, "tensor matmul launch");
     return RK_OK;
 }
-
-static unsigned elem_grid(int64_t n) { return (unsigned)std::min<int64_t>((n + 255) / 256, 65536); }
 
 int enqueue_tensor_quantize(rk_device *d, const float *a, int8_t *q, int64_t n, float k, hipStream_t s) {
     ProfScope p(d, s, "tensor_quantize");

@@ -102,3 +102,52 @@ def test_argument_errors(dev):
         dev.tensor_quantize(f, 0.0)
     with pytest.raises(rkhip.RKError):
         dev.tensor_scale(np.ones(3, np.int8), 1.0)
+
+
+# Sizes about the tiles' edges (32 outputs a side in f32; 128, 64 and 32 in
+# i8, by the number of tiles), the staged slices' (64 positions; 128, 256 and
+# 512) and the loads' (4 floats, 16 bytes), on host buffers and on device
+# pointers off their alignment.
+TILE_SHAPES = [(32, 64, 32), (33, 65, 31), (31, 63, 97), (1, 1, 1), (2, 15, 3), (64, 128, 260), (513, 17, 65),
+               (300, 130, 70)]
+
+
+@pytest.mark.parametrize("m,k,n", TILE_SHAPES + [(1024, 48, 1030)])
+def test_f32_tiles(dev, m, k, n):
+    rng = np.random.default_rng(m + 31 * k + 7 * n)
+    a = awkward(rng, m * k, 1.0).reshape(m, k)
+    b = awkward(rng, k * n, 1.0).reshape(k, n)
+    want = bits(oracle.tensor_matmul_f32(a, b, False))
+    assert np.array_equal(bits(dev.tensor_matmul(a, b)), want)
+    assert np.array_equal(bits(dev.tensor_matmul(a, np.ascontiguousarray(b.T), transposed=True)), want)
+
+
+@pytest.mark.parametrize("m,k,n", TILE_SHAPES + [(70, 511, 33), (70, 513, 31), (1000, 257, 700), (1025, 16, 1021),
+                                                 (2048, 129, 1600), (1793, 143, 1795)])
+@pytest.mark.parametrize("off", [0, 1, 6])
+def test_i8_tiles(dev, m, k, n, off):
+    rng = np.random.default_rng(m + 31 * k + 7 * n)
+    a = rng.integers(-128, 128, (m, k), dtype=np.int16).astype(np.int8)
+    b = rng.integers(-128, 128, (k, n), dtype=np.int16).astype(np.int8)
+    want = oracle.tensor_matmul_i8(a, b, False)
+
+    def words(v):  # the bytes, `off` bytes into their words
+        v = np.concatenate((np.zeros(off, np.int8), v.ravel()))
+        return np.concatenate((v, np.zeros(-v.size % 4, np.int8))).view(np.float32)
+
+    at_a, at_b, at_c = 0, words(a).size, words(a).size + words(b).size
+    arena = dev.arena(at_c + m * n, at_c + m * n)
+    for transposed, y in ((0, b), (1, np.ascontiguousarray(b.T))):
+        q = arena.begin()
+        q.write(at_a, words(a))
+        q.write(at_b, words(y))
+        q.write(at_c, np.full(m * n, -1, np.int32).view(np.float32))
+        q.submit()
+        dev._check(rkhip.lib().rk_tensor_matmul_device(dev.h, rkhip.TENSOR_I8, transposed, m, k, n,
+                                                       arena.device_ptr(at_a) + off, arena.device_ptr(at_b) + off,
+                                                       arena.device_ptr(at_c), None))
+        q = arena.begin()
+        got = q.read(at_c, m * n)
+        q.submit()
+        assert np.array_equal(got.view(np.int32).reshape(m, n), want)
+    arena.free()
