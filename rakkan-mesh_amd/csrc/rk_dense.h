@@ -9,10 +9,17 @@ namespace rk {
 // up to a multiple of 32, the padding zero.
 int64_t dense_row_elems(int64_t cols);
 
-// out[r] = Dot32(row r, x) for r < rows (internal/num/matvec.go:106-123
-// MatVec32 / MatVecBF16): w holds rows of dense_row_elems(cols) float32
-// (bf16 false) or bfloat16 (bf16 true) values; x and out device buffers.
-void launch_dense_matvec(bool bf16, const void *w, int64_t rows, int64_t cols, const float *x, float *out,
-                         hipStream_t s);
+// One product of a launch: out[r] = Dot32(row r, x) for r < rows
+// (internal/num/matvec.go:106-123 MatVec32 / MatVecBF16); w holds rows of
+// dense_row_elems(cols) float32 or bfloat16 values, device buffers.
+struct DenseMat {
+    const void *w;
+    float *out;
+    int64_t rows;
+};
+constexpr int kDenseMats = 3;  // matrices of a launch
+
+// n (<= kDenseMats) matrices of one format times x (cols device floats).
+void launch_dense_matvecs(bool bf16, const DenseMat *m, int n, int64_t cols, const float *x, hipStream_t s);
 
 }  // namespace rk

@@ -14,16 +14,23 @@
 // never become -0 (x + y is -0 only when both are), so s + (+0) == s, NaN
 // payloads included.
 //
-// Work layout: 32/SL lanes per row; lane l of a row keeps the running sums
-// SL·l .. SL·l+SL-1 and at row step m (32 elements) reads elements
-// 32m+SL·l .. +SL-1, so a row step is one contiguous 128-byte (float32) or
-// 64-byte (bfloat16) segment. U steps of every row are in flight (a
-// register ring). The row's loads are buffer loads at a wave-uniform step
-// offset; past the row's last step they repeat that step (cache hits) and
-// those steps add +0, so every step issues the same loads and additions and
-// the waits are fixed counts. The input is staged in LDS (zero-padded), in
-// segments of kDenseMaxLdsElems for wider rows, and read a block of U steps
-// at a time.
+// Work layout: 32 lanes per row, two rows a wave; lane l of a row keeps the
+// running sum l and takes element 32m + l of row step m. A wave's rows come
+// by direct-to-LDS loads, 1 KiB of one row an instruction, into a ring of
+// its own of kDenseRing parts of 16 steps: the bytes in flight need no
+// registers, many waves fit a CU, and a part is waited for by count, without
+// a barrier. The input is staged in LDS the same way (kDenseX elements at a
+// time for wider rows). Up to three matrices of one input share a launch.
+//
+// What bounds it: HBM, then the launch and the input's way into LDS for the
+// smaller ones. MI355X, bfloat16 (us, weights past the MALL; before: rows
+// loaded a step an instruction into registers, a launch a matrix):
+// 2048 + 512 + 512 x 2048 5.3 (24.3), 8192 + 8192 x 2048 12.9, 5.2 TB/s
+// (21.5), 2048 x 8192 9.7 (21.4), 4096 x 4096 8.7 (12.0), 14336 + 14336 x
+// 4096 41.3, 5.7 TB/s (57.0); float32 23.2 (29.9), 15.1 (18.3), 13.3 (15.1)
+// and 72.0, 6.5 TB/s (80.5) for the last four. Rings of 3, 4 and 8 parts
+// were slower (8192 + 8192: 14.0, 14.9, 20.1: fewer waves fit), as were two
+// sums a lane, four rows a wave (15.5) and 1, 2 and 8 waves a workgroup.
 #include <algorithm>
 #include <mutex>
 
@@ -35,210 +42,233 @@ namespace rk {
 
 namespace {
 
-// Running sums per lane (32/SL lanes a row) and row steps in flight, the
-// fastest measured on MI355X: float32 one sum a lane (4-byte loads, two
-// rows a wave), bfloat16 two (one 4-byte word, four rows a wave).
-constexpr int kDenseSlF32 = 1;
-constexpr int kDenseSlBf16 = 2;
-constexpr int kDenseU = 16;
-constexpr int kDenseMaxLdsElems = 32768;    // input staged in LDS up to this width (128 KiB)
-constexpr int64_t kDenseLaunchBytes = 1 << 30;  // a launch's matrix bytes (one buffer resource)
+constexpr int kDensePart = 512;  // elements of a row (16 steps) in a ring part
+constexpr int kDenseX = 8192;    // input elements staged at a time
+constexpr int kDenseRing = 2;    // parts of a wave's ring
 
 typedef int rk_v2i __attribute__((ext_vector_type(2)));
+typedef float rk_v2f __attribute__((ext_vector_type(2)));
+typedef float rk_v4f __attribute__((ext_vector_type(4)));
 
-// Lanes per row 32/SL: lane l of a row keeps running sums SL·l .. SL·l+SL-1
-// and reads SL elements per row step. U row steps in flight (U <= 63, the
-// vector memory counter's range).
-template <bool BF, int SL>
-struct DenseLoad;
-template <>
-struct DenseLoad<false, 1> {
-    typedef int type;
-    static __device__ type load(__amdgpu_buffer_rsrc_t r, int v, int s) {
-        return __builtin_amdgcn_raw_buffer_load_b32(r, v, s, kAuxStream);
-    }
-};
-template <>
-struct DenseLoad<false, 2> {
-    typedef rk_v2i type;
-    static __device__ type load(__amdgpu_buffer_rsrc_t r, int v, int s) {
-        return __builtin_amdgcn_raw_buffer_load_b64(r, v, s, kAuxStream);
-    }
-};
-template <>
-struct DenseLoad<false, 4> {
-    typedef rk_v4i type;
-    static __device__ type load(__amdgpu_buffer_rsrc_t r, int v, int s) {
-        return __builtin_amdgcn_raw_buffer_load_b128(r, v, s, kAuxStream);
-    }
-};
-template <>
-struct DenseLoad<true, 2> {
-    typedef int type;
-    static __device__ type load(__amdgpu_buffer_rsrc_t r, int v, int s) {
-        return __builtin_amdgcn_raw_buffer_load_b32(r, v, s, kAuxStream);
-    }
-};
-template <>
-struct DenseLoad<true, 4> {
-    typedef rk_v2i type;
-    static __device__ type load(__amdgpu_buffer_rsrc_t r, int v, int s) {
-        return __builtin_amdgcn_raw_buffer_load_b64(r, v, s, kAuxStream);
-    }
+struct DenseArgs {
+    DenseMat m[kDenseMats];
+    int64_t first[kDenseMats];  // a matrix's first wave
+    const float *x;
+    int64_t row_elems;
+    int32_t cols, waves;        // waves a workgroup
 };
 
-// Element k (< SL) of a loaded step as float32.
-template <bool BF, int SL, typename V>
-__device__ __forceinline__ float dense_elem(const V &v, int k) {
-    if constexpr (!BF) {
-        if constexpr (SL == 1)
-            return __int_as_float(v);
-        else
-            return __int_as_float(v[k]);
-    } else {
-        int word;
-        if constexpr (SL == 2)
-            word = v;
-        else
-            word = v[k >> 1];
-        return __int_as_float((k & 1) ? (word & (int)0xFFFF0000u) : (word << 16));
-    }
+__device__ __forceinline__ uint32_t lds_off(void *p) { return (uint32_t)(uintptr_t)lds_ptr(p); }
+
+// 16 bytes a lane from global memory into LDS at `to` + 16·lane.
+__device__ __forceinline__ void load_lds16(const uint8_t *from, uint8_t *to) {
+    __builtin_amdgcn_global_load_lds(from, lds_ptr(to), 16, 0, kAuxStream);
 }
 
-template <bool BF, int SL, int U>
-__global__ __launch_bounds__(512) void dense_matvec_kernel(const void *w, int64_t rows, int row_elems,
-                                                            const float *x, int cols, float *out) {
-    typedef DenseLoad<BF, SL> LD;
-    typedef typename LD::type V;
-    constexpr int LPR = 32 / SL;    // lanes per row
-    constexpr int RPW = 64 / LPR;   // rows per wave
-    constexpr int ES = BF ? 2 : 4;  // bytes per element
-    constexpr int SB = 32 * ES;     // bytes per row step
-    extern __shared__ __align__(16) float sx[];
-    const int tid = threadIdx.x, lane = tid & 63, l = lane % LPR;
-    const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + (tid >> 6);
-    const int64_t row = wave * RPW + lane / LPR;
-    // groups past the end repeat the last row (never stored) and take part
-    // in the workgroup's barriers
-    const int64_t r = row < rows ? row : rows - 1;
-    const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(w), 0, (int)(rows * row_elems * ES), kRsrcWord3);
-    const int vo = (int)(r * row_elems * ES) + l * SL * ES;
-    float acc[SL];
-#pragma unroll
-    for (int k = 0; k < SL; k++) acc[k] = 0.0f;
-    // segments of the row whose input fits the LDS (one for widths up to
-    // kDenseMaxLdsElems)
-    for (int c0 = 0; c0 < row_elems; c0 += kDenseMaxLdsElems) {  // uniform
-        const int ce = min(kDenseMaxLdsElems, row_elems - c0);
-        const int nsteps = ce >> 5, mb = c0 >> 5;
-        auto load = [&](int m) -> V { return LD::load(rs, vo, (mb + (m < nsteps ? m : nsteps - 1)) * SB); };
-        // the segment's first U steps, oldest first (the ring's waits count
-        // on that order), then its input into LDS, zero past cols
-        V wb[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            wb[u] = load(u);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (c0 > 0) __syncthreads();  // every wave is done with the previous segment's input
-        for (int i = tid; i < ce; i += blockDim.x) sx[i] = c0 + i < cols ? x[c0 + i] : 0.0f;
-        __syncthreads();
-        for (int m0 = 0; m0 < nsteps; m0 += U) {
-            // the block's U input steps from LDS first (one LDS latency a
-            // block, not a step)
-            float xv[U][SL];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int m = m0 + u;
-                const float *xp = sx + (m < nsteps ? m : nsteps - 1) * 32 + l * SL;
-                if constexpr (SL == 4) {
-                    const float4 t = *reinterpret_cast<const float4 *>(xp);
-                    xv[u][0] = t.x, xv[u][1] = t.y, xv[u][2] = t.z, xv[u][3] = t.w;
-                } else if constexpr (SL == 2) {
-                    const float2 t = *reinterpret_cast<const float2 *>(xp);
-                    xv[u][0] = t.x, xv[u][1] = t.y;
-                } else {
-                    xv[u][0] = xp[0];
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                // every step adds (no branch, so no load is left in flight
-                // under a register it is about to reload); a step past the
-                // segment adds +0, which leaves the sum as it is
-                const int m = m0 + u;
-                const bool live = m < nsteps;  // uniform
-#pragma unroll
-                for (int k = 0; k < SL; k++)
-                    acc[k] += live ? dense_elem<BF, SL>(wb[u], k) * xv[u][k] : 0.0f;
-                wb[u] = load(m + U);
-            }
-        }
+// Waits until at most n·NI of the wave's loads are in flight (n <= 7).
+template <int NI>
+__device__ __forceinline__ void wait_parts(int n) {
+    switch (n) {  // uniform
+    case 0: __builtin_amdgcn_s_waitcnt(vmcnt_wait(0)); break;
+    case 1: __builtin_amdgcn_s_waitcnt(vmcnt_wait(NI)); break;
+    case 2: __builtin_amdgcn_s_waitcnt(vmcnt_wait(2 * NI)); break;
+    case 3: __builtin_amdgcn_s_waitcnt(vmcnt_wait(3 * NI)); break;
+    case 4: __builtin_amdgcn_s_waitcnt(vmcnt_wait(4 * NI)); break;
+    case 5: __builtin_amdgcn_s_waitcnt(vmcnt_wait(5 * NI)); break;
+    case 6: __builtin_amdgcn_s_waitcnt(vmcnt_wait(6 * NI)); break;
+    default: __builtin_amdgcn_s_waitcnt(vmcnt_wait(7 * NI)); break;
     }
-    // Dot32's combine: s_j sits in lane j/SL of the row, element j mod SL.
-    // a = s_j + s_j+8 (lanes of j < 8), then + (s_j+16 + s_j+24) gives e_j;
-    // then ((e0+e1)+(e2+e3))+((e4+e5)+(e6+e7)).
-    float e[SL];
-#pragma unroll
-    for (int k = 0; k < SL; k++) {
-        const float a = acc[k] + __shfl_down(acc[k], 8 / SL, LPR);
-        e[k] = a + __shfl_down(a, 16 / SL, LPR);
-    }
-    // lanes 0 .. 8/SL-1 hold e_j (j = SL·l + k)
-    float res;
-    if constexpr (SL == 4) {
-        const float h = (e[0] + e[1]) + (e[2] + e[3]);  // lane 0: e0..e3; lane 1: e4..e7
-        res = h + __shfl_down(h, 1, LPR);
-    } else if constexpr (SL == 2) {
-        const float p = e[0] + e[1];                    // lane l: e_2l + e_2l+1
-        const float t = p + __shfl_down(p, 1, LPR);     // lanes 0, 2
-        res = t + __shfl_down(t, 2, LPR);
-    } else {
-        const float p = e[0] + __shfl_down(e[0], 1, LPR);  // lanes 0, 2, 4, 6
-        const float t = p + __shfl_down(p, 2, LPR);        // lanes 0, 4
-        res = t + __shfl_down(t, 4, LPR);
-    }
-    if (l == 0 && row < rows) out[row] = res;
+    asm volatile("" ::: "memory");
 }
 
-template <bool BF, int SL, int U>
-void launch_dense_t(const void *w, int64_t rows, int row_elems, const float *x, int cols, float *out,
-                    hipStream_t s, int waves_per_wg = 0) {
-    constexpr int RPW = 2 * SL;
-    const size_t lds = (size_t)std::min(row_elems, kDenseMaxLdsElems) * 4;
+// A part's 16 steps of a lane from LDS: weights at byte wa (step stride 64 or
+// 128), input at byte xa (step stride 128). The reads and their wait are one
+// block, so no output is seen before it has arrived (and the compiler, which
+// cannot tell the ring's parts apart, adds no wait for the loads in flight).
+template <bool BF>
+struct DensePart;
+template <>
+struct DensePart<true> {
+    int w[16];
+    rk_v2f x[8];
+    __device__ __forceinline__ void read(uint32_t wa, uint32_t xa) {
+        asm volatile(
+            "ds_read_u16 %0, %24\n\tds_read_u16 %1, %24 offset:64\n\tds_read2_b32 %16, %25 offset0:0 offset1:32\n\t"
+            "ds_read_u16 %2, %24 offset:128\n\tds_read_u16 %3, %24 offset:192\n\tds_read2_b32 %17, %25 offset0:64 offset1:96\n\t"
+            "ds_read_u16 %4, %24 offset:256\n\tds_read_u16 %5, %24 offset:320\n\tds_read2_b32 %18, %25 offset0:128 offset1:160\n\t"
+            "ds_read_u16 %6, %24 offset:384\n\tds_read_u16 %7, %24 offset:448\n\tds_read2_b32 %19, %25 offset0:192 offset1:224\n\t"
+            "ds_read_u16 %8, %24 offset:512\n\tds_read_u16 %9, %24 offset:576\n\tds_read2_b32 %20, %26 offset0:0 offset1:32\n\t"
+            "ds_read_u16 %10, %24 offset:640\n\tds_read_u16 %11, %24 offset:704\n\tds_read2_b32 %21, %26 offset0:64 offset1:96\n\t"
+            "ds_read_u16 %12, %24 offset:768\n\tds_read_u16 %13, %24 offset:832\n\tds_read2_b32 %22, %26 offset0:128 offset1:160\n\t"
+            "ds_read_u16 %14, %24 offset:896\n\tds_read_u16 %15, %24 offset:960\n\tds_read2_b32 %23, %26 offset0:192 offset1:224\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4]), "=&v"(w[5]), "=&v"(w[6]), "=&v"(w[7]),
+              "=&v"(w[8]), "=&v"(w[9]), "=&v"(w[10]), "=&v"(w[11]), "=&v"(w[12]), "=&v"(w[13]), "=&v"(w[14]),
+              "=&v"(w[15]), "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]), "=&v"(x[5]), "=&v"(x[6]),
+              "=&v"(x[7])
+            : "v"(wa), "v"(xa), "v"(xa + 1024)
+            : "memory");
+    }
+    __device__ __forceinline__ float weight(int m) const { return __int_as_float(w[m] << 16); }
+    __device__ __forceinline__ float input(int m) const { return x[m >> 1][m & 1]; }
+};
+template <>
+struct DensePart<false> {
+    rk_v2f w[8], x[8];
+    __device__ __forceinline__ void read(uint32_t wa, uint32_t xa) {
+        asm volatile(
+            "ds_read2_b32 %0, %16 offset0:0 offset1:32\n\tds_read2_b32 %8, %18 offset0:0 offset1:32\n\t"
+            "ds_read2_b32 %1, %16 offset0:64 offset1:96\n\tds_read2_b32 %9, %18 offset0:64 offset1:96\n\t"
+            "ds_read2_b32 %2, %16 offset0:128 offset1:160\n\tds_read2_b32 %10, %18 offset0:128 offset1:160\n\t"
+            "ds_read2_b32 %3, %16 offset0:192 offset1:224\n\tds_read2_b32 %11, %18 offset0:192 offset1:224\n\t"
+            "ds_read2_b32 %4, %17 offset0:0 offset1:32\n\tds_read2_b32 %12, %19 offset0:0 offset1:32\n\t"
+            "ds_read2_b32 %5, %17 offset0:64 offset1:96\n\tds_read2_b32 %13, %19 offset0:64 offset1:96\n\t"
+            "ds_read2_b32 %6, %17 offset0:128 offset1:160\n\tds_read2_b32 %14, %19 offset0:128 offset1:160\n\t"
+            "ds_read2_b32 %7, %17 offset0:192 offset1:224\n\tds_read2_b32 %15, %19 offset0:192 offset1:224\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4]), "=&v"(w[5]), "=&v"(w[6]), "=&v"(w[7]),
+              "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]), "=&v"(x[5]), "=&v"(x[6]), "=&v"(x[7])
+            : "v"(wa), "v"(wa + 1024), "v"(xa), "v"(xa + 1024)
+            : "memory");
+    }
+    __device__ __forceinline__ float weight(int m) const { return w[m >> 1][m & 1]; }
+    __device__ __forceinline__ float input(int m) const { return x[m >> 1][m & 1]; }
+};
+
+template <bool BF>
+struct DenseShape {
+    static constexpr int RPW = 2;  // rows a wave
+    static constexpr int ES = BF ? 2 : 4, SB = 32 * ES;  // bytes an element, a row step
+    static constexpr int PB = kDensePart * ES;           // bytes of a row in a part
+    // rows of a part lie PB + pad apart, so a step's pieces fall in distinct banks
+    static constexpr int PITCH = PB + (BF ? 64 : 128), PART = RPW * PITCH;
+    static constexpr int NI = RPW * (PB / 1024);         // loads a part
+};
+
+template <bool BF>
+__global__ __launch_bounds__(256) void dense_matvec_kernel(DenseArgs a) {
+    typedef DenseShape<BF> D;
+    constexpr int S = kDenseRing;
+    extern __shared__ __align__(16) uint8_t dense_lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l = lane & 31, g = lane >> 5;
+    const int re = (int)a.row_elems;
+    const int xe = min(re, kDenseX);  // input elements staged at a time
+    float *sx = reinterpret_cast<float *>(dense_lds);
+    uint8_t *ring = dense_lds + 4 * ((xe + kDensePart - 1) / kDensePart * kDensePart) + wv * S * D::PART;
+    // the wave's matrix and rows; past the end it repeats the last row
+    // (never stored) and takes part in the barriers
+    const int64_t gw = (int64_t)blockIdx.x * a.waves + wv;
+    const int mi = (gw >= a.first[1] ? 1 : 0) + (gw >= a.first[2] ? 1 : 0);
+    const uint8_t *w = static_cast<const uint8_t *>(a.m[mi].w);
+    const int64_t rows = a.m[mi].rows, r0 = (gw - a.first[mi]) * D::RPW;
+    const int64_t rb = (int64_t)re * D::ES;
+    const int parts = (re + kDensePart - 1) / kDensePart;
+    // part c into its place in the ring; past the row's end the last 16
+    // bytes again (never added)
+    auto fetch = [&](int c) {
+        uint8_t *to = ring + (c % S) * D::PART;
+#pragma unroll
+        for (int r = 0; r < D::RPW; r++) {
+            const uint8_t *row = w + min(r0 + r, rows - 1) * rb;
+#pragma unroll
+            for (int h = 0; h < D::PB / 1024; h++)
+                load_lds16(row + min((int64_t)c * D::PB + 1024 * h + 16 * lane, rb - 16), to + r * D::PITCH + 1024 * h);
+        }
+    };
+    // input elements c0 .. c0 + n, zeros past cols
+    const bool a16 = ((uintptr_t)a.x & 15) == 0;
+    auto stage = [&](int c0) {
+        const int n = min(xe, re - c0), have = max(0, min(n, a.cols - c0)), m16 = a16 ? have & ~255 : 0;
+        const float *x = a.x + c0;
+        for (int p = 256 * wv; p < m16; p += 256 * a.waves)
+            __builtin_amdgcn_global_load_lds(x + p + 4 * lane, lds_ptr(sx + p), 16, 0, 0);
+        for (int p = m16 + 64 * wv; p + 64 <= have; p += 64 * a.waves)
+            __builtin_amdgcn_global_load_lds(x + p + lane, lds_ptr(sx + p), 4, 0, 0);
+        const int t = (have & ~63) + lane;  // fewer than 64 left, then zeros
+        if (wv == 0 && t < n) sx[t] = t < have ? x[t] : 0.0f;
+    };
+    stage(0);
+    const int ahead = min(S, parts);
+    for (int c = 0; c < ahead; c++) fetch(c);
+    // the input is there once only the weights' loads are in flight
+    static_assert(S * D::NI <= 63, "the counter's range");
+    if (ahead == S)
+        __builtin_amdgcn_s_waitcnt(vmcnt_wait(S * D::NI));
+    else
+        __builtin_amdgcn_s_waitcnt(vmcnt_wait(0));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    const uint32_t wo = lds_off(ring) + g * D::PITCH + l * D::ES, xo = lds_off(sx) + 4 * l;
+    float acc = 0.0f;
+    for (int c = 0; c < parts; c++) {
+        const int e0 = c * kDensePart, c0 = e0 % kDenseX;
+        if (c0 == 0 && c > 0) {  // the next elements of a wide row's input
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();  // every wave is done with the last ones
+            stage(e0);
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+        }
+        wait_parts<D::NI>(min(S - 1, parts - 1 - c));
+        DensePart<BF> t;
+        t.read(wo + (c % S) * D::PART, xo + 4 * c0);
+        if (c + S < parts) fetch(c + S);  // into the part just read
+        if (e0 + kDensePart <= re) {
+#pragma unroll
+            for (int m = 0; m < 16; m++) acc += t.weight(m) * t.input(m);
+        } else {
+#pragma unroll
+            for (int m = 0; m < 16; m++)
+                if (e0 + 32 * m < re) acc += t.weight(m) * t.input(m);  // uniform
+        }
+    }
+    // Dot32's combine, s_j in lane j of the row: s_j + s_j+8 (lanes of j <
+    // 8), then + (s_j+16 + s_j+24) gives e_j; then
+    // ((e0+e1)+(e2+e3))+((e4+e5)+(e6+e7)).
+    const float v = acc + __shfl_down(acc, 8, 32);
+    const float e = v + __shfl_down(v, 16, 32);
+    const float p = e + __shfl_down(e, 1, 32);  // lanes 0, 2, 4, 6
+    const float q = p + __shfl_down(p, 2, 32);  // lanes 0, 4
+    const float res = q + __shfl_down(q, 4, 32);
+    if (l == 0 && r0 + g < rows) a.m[mi].out[r0 + g] = res;
+}
+
+template <bool BF>
+void launch_dense_t(DenseArgs a, int n, hipStream_t s) {
+    typedef DenseShape<BF> D;
     static std::once_flag once;
     std::call_once(once, [] {
-        (void)hipFuncSetAttribute((const void *)dense_matvec_kernel<BF, SL, U>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, kDenseMaxLdsElems * 4);
+        (void)hipFuncSetAttribute((const void *)dense_matvec_kernel<BF>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  4 * kDenseX + 4 * kDenseRing * D::PART);
     });
-    const int64_t waves = (rows + RPW - 1) / RPW;
-    // four waves a workgroup once there are enough (measured best on
-    // MI355X for 4096- and 14336-row products)
-    const int64_t W = waves_per_wg > 0 ? waves_per_wg : std::min<int64_t>(4, std::max<int64_t>(1, waves / 256));
-    const int64_t grid = (waves + W - 1) / W;
-    RK_LAUNCH((dense_matvec_kernel<BF, SL, U>), dim3((unsigned)grid), dim3((unsigned)(64 * W)), lds, s, w, rows,
-              row_elems, x, cols, out);
+    int64_t waves = 0;
+    for (int i = 0; i < kDenseMats; i++) {
+        a.first[i] = i < n ? waves : INT64_MAX;
+        if (i < n) waves += (a.m[i].rows + D::RPW - 1) / D::RPW;
+    }
+    // four waves a workgroup once that leaves every CU a workgroup
+    a.waves = (int)std::min<int64_t>(4, std::max<int64_t>(1, waves / 256));
+    const int64_t xe = (std::min<int64_t>(a.row_elems, kDenseX) + kDensePart - 1) / kDensePart * kDensePart;
+    const size_t lds = (size_t)(4 * xe + a.waves * kDenseRing * D::PART);
+    RK_LAUNCH(dense_matvec_kernel<BF>, dim3((unsigned)((waves + a.waves - 1) / a.waves)),
+              dim3((unsigned)(64 * a.waves)), lds, s, a);
 }
 
 }  // namespace
 
 int64_t dense_row_elems(int64_t cols) { return (cols + 31) & ~(int64_t)31; }
 
-void launch_dense_matvec(bool bf16, const void *w, int64_t rows, int64_t cols, const float *x, float *out,
-                         hipStream_t s) {
-    const int row_elems = (int)dense_row_elems(cols);
-    const int64_t rb = (int64_t)row_elems * (bf16 ? 2 : 4);
-    const int64_t per = std::max<int64_t>(1, kDenseLaunchBytes / rb);  // rows of one launch
-    for (int64_t r0 = 0; r0 < rows; r0 += per) {
-        const int64_t n = std::min(per, rows - r0);
-        const void *wr = static_cast<const uint8_t *>(w) + r0 * rb;
-        if (bf16)
-            launch_dense_t<true, kDenseSlBf16, kDenseU>(wr, n, row_elems, x, (int)cols, out + r0, s);
-        else
-            launch_dense_t<false, kDenseSlF32, kDenseU>(wr, n, row_elems, x, (int)cols, out + r0, s);
-    }
+void launch_dense_matvecs(bool bf16, const DenseMat *m, int n, int64_t cols, const float *x, hipStream_t s) {
+    DenseArgs a{};
+    a.x = x;
+    a.row_elems = dense_row_elems(cols);
+    a.cols = (int32_t)cols;
+    for (int i = 0; i < n; i++) a.m[i] = m[i];
+    if (bf16)
+        launch_dense_t<true>(a, n, s);
+    else
+        launch_dense_t<false>(a, n, s);
 }
 
 }  // namespace rk

@@ -178,11 +178,22 @@ int enqueue_matvecs(rk_device *d, int32_t n, rk_matrix *const *ms, float *const 
                          reinterpret_cast<const uint8_t *>(q.qx), q.xs, outs[i], ms[i]->raw != 0, s);
     }
     // float32 / bfloat16 matrices take x as it is (internal/gpu/batch.go:
-    // 263-264: no quantized input), one launch each
-    for (int i = 0; i < n; i++) {
-        if (ms[i]->kind != RK_F32 && ms[i]->kind != RK_BF16) continue;
-        ProfScope p(d, s, ms[i]->kind == RK_BF16 ? "matvec_bf16" : "matvec_f32");
-        launch_dense_matvec(ms[i]->kind == RK_BF16, ms[i]->w, ms[i]->rows, cols, x, outs[i], s);
+    // 263-264: no quantized input), up to three of a format a launch
+    for (int kind : {RK_F32, RK_BF16}) {
+        DenseMat dm[kDenseMats];
+        int k = 0;
+        auto flush = [&]() {
+            if (k == 0) return;
+            ProfScope p(d, s, kind == RK_BF16 ? "matvec_bf16" : "matvec_f32");
+            launch_dense_matvecs(kind == RK_BF16, dm, k, cols, x, s);
+            k = 0;
+        };
+        for (int i = 0; i < n; i++) {
+            if (ms[i]->kind != kind) continue;
+            dm[k++] = DenseMat{ms[i]->w, outs[i], ms[i]->rows};
+            if (k == kDenseMats) flush();
+        }
+        flush();
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(d, e, "matvec launch");

@@ -151,3 +151,39 @@ def test_dense_shape_errors(dev):
     finally:
         m.free()
     assert dev.used == 0
+
+
+# Widths about the ring's parts (512 elements), the pieces the input is
+# staged in (64 and 256) and the elements staged at a time (8192); four
+# matrices of a call take two launches, of odd row counts (two rows a wave,
+# one to four waves a workgroup); an input off its 16-byte alignment.
+@pytest.mark.parametrize("cols", [2, 62, 254, 256, 320, 510, 512, 514, 1056, 2048, 8190, 8192, 8194, 16416])
+@pytest.mark.parametrize("kind", [rkhip.F32, rkhip.BF16])
+def test_dense_parts(dev, kind, cols):
+    rng = np.random.default_rng(cols + kind)
+    rows = [1, 5, 1030, 3] if cols <= 1056 else [3, 130, 2, 1]
+    x = awkward(rng, cols)
+    ws = [awkward(rng, r * cols, 0.1) for r in rows]
+    if kind == rkhip.BF16:
+        ws = [to_bf16(w) for w in ws]
+    ms = [dev.upload(kind, r, cols, w) for r, w in zip(rows, ws)]
+    ref = oracle.matvec32 if kind == rkhip.F32 else oracle.matvec_bf16
+    want = [ref(w, x, r, cols) for r, w in zip(rows, ws)]
+    offs = np.cumsum([cols + 4] + rows).tolist()
+    arena = dev.arena(offs[-1], offs[-1])
+    try:
+        for got, w in zip(dev.matvecs(ms, x), want):
+            same_bits(got, w, f"{cols} columns")
+        for at in (0, 1, 3):
+            b = arena.begin()
+            b.write(at, x)
+            b.matvecs(ms, offs[:4], at)
+            got = [b.read(o, r) for o, r in zip(offs, rows)]
+            b.submit()
+            for y, w in zip(got, want):
+                same_bits(np.asarray(y), w, f"{cols} columns, input at word {at}")
+    finally:
+        arena.free()
+        for m in ms:
+            m.free()
+    assert dev.used == 0
