@@ -14,6 +14,9 @@
 // a workgroup runs sixteen tokens' sequential sums side by side (one per
 // half-wave for the softmax, one per lane and element for the values, a
 // lane holding the elements e, e+32, e+64, e+96 of its token).
+//
+// Several sequences' prompts in one batch (AttBatch::groups): a group is a
+// run of one sequence's tokens, over that sequence's caches.
 #include <mutex>
 
 #include "rk_dev.h"
@@ -23,7 +26,7 @@ namespace rk {
 
 namespace {
 
-constexpr int kGrpTok = 16;    // tokens per workgroup
+constexpr int kGrpTok = kAttGroupTok;  // tokens per workgroup
 constexpr int kGrpMaxT = 1024;  // positions a group's weights keep in LDS
 constexpr int kScTile = 64;    // positions per scores workgroup
 // The values workgroup's shape: SL 32-element slices of a head (SL = 4, or
@@ -36,6 +39,20 @@ constexpr int kScTile = 64;    // positions per scores workgroup
     constexpr int kGvPitch = kGvChunk + 4;           /* floats per element row (odd count of 16-byte units) */
 constexpr int kGvThreads = 512;         // eight waves, two tokens each
 constexpr int kHs = 128;                // head size of the scores kernel
+
+// Group i of a batch: its tokens, its first token's position, its caches.
+struct GrpRows {
+    int z0, nz, pos0;
+    int64_t cache0;
+};
+__device__ __forceinline__ GrpRows group_rows(const AttBatch &bt, int i) {
+    if (bt.groups) {
+        const AttGroup g = bt.groups[i];
+        return GrpRows{g.row0, g.n, g.pos0, g.seq * bt.cache_stride};
+    }
+    const int z0 = i * kGrpTok;
+    return GrpRows{z0, min(kGrpTok, bt.tokens - z0), bt.pos0 + z0, 0};
+}
 
 // acc[s] + Σ a[t]·v_s[t] for t < n in order, for the SL rows v_s = v +
 // 32·s·kGvPitch (float32; each product rounded, then added), a and v in LDS
@@ -93,9 +110,9 @@ __global__ __launch_bounds__(256) void att_scores_group_kernel(const float *q, c
     __shared__ __align__(16) float sq[kGrpTok][kHs];
     const int h = blockIdx.x, g = h / kv_mul;
     const int t0 = blockIdx.y * kScTile;
-    const int z0 = blockIdx.z * kGrpTok;
-    const int nz = min(kGrpTok, bt.tokens - z0);
-    const int tmax = bt.pos0 + z0 + nz;  // positions the group's last token sees
+    const GrpRows gr = group_rows(bt, blockIdx.z);
+    const int z0 = gr.z0, nz = gr.nz;
+    const int tmax = gr.pos0 + nz;  // positions the group's last token sees
     if (t0 >= tmax) return;
     const int part = threadIdx.x & 3;
     const int t = t0 + (threadIdx.x >> 2);
@@ -104,7 +121,7 @@ __global__ __launch_bounds__(256) void att_scores_group_kernel(const float *q, c
         reinterpret_cast<float4 *>(&sq[zl][0])[e4] = reinterpret_cast<const float4 *>(
             q + (int64_t)(z0 + min(zl, nz - 1)) * bt.q_stride + (int64_t)h * kHs)[e4];
     }
-    const float *kt = keys + (int64_t)min(t, tmax - 1) * kv_dim + (int64_t)g * kHs;
+    const float *kt = keys + gr.cache0 + (int64_t)min(t, tmax - 1) * kv_dim + (int64_t)g * kHs;
     float4 k0[kHs / 32], k1[kHs / 32];
 #pragma unroll
     for (int st = 0; st < kHs / 32; st++) {
@@ -137,7 +154,7 @@ __global__ __launch_bounds__(256) void att_scores_group_kernel(const float *q, c
         }
         const float dot = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
         const int z = z0 + zl;
-        if (part == 0 && t < bt.pos0 + z + 1)
+        if (part == 0 && t < gr.pos0 + zl + 1)
             att[(int64_t)z * bt.att_stride + (int64_t)h * att_stride + t] = dot * inv_sqrt;
     }
 }
@@ -163,19 +180,19 @@ __global__ __launch_bounds__(kGvThreads) void att_values_group_kernel(const floa
     const int ns = min(kGvSlices, (hs - e0) >> 5);  // slices of the head here
     // the last token groups (the most positions) are dispatched first, so
     // the short ones fill the machine's last round
-    const int z0 = (int)(gridDim.z - 1 - blockIdx.z) * kGrpTok;
-    const int nz = min(kGrpTok, bt.tokens - z0);
+    const GrpRows gr = group_rows(bt, (int)(gridDim.z - 1 - blockIdx.z));
+    const int z0 = gr.z0, nz = gr.nz;
     const int zl = 2 * wave + (lane >> 5), l32 = lane & 31;
     const int zc = min(zl, nz - 1);      // halves past the batch repeat its last token, unstored
-    const int Tz = bt.pos0 + z0 + zc + 1;
-    const int tmax = bt.pos0 + z0 + nz;
+    const int Tz = gr.pos0 + zc + 1;
+    const int tmax = gr.pos0 + nz;
     float *az = sa + zl * apitch;
 
     // ---- the value tiles' loads: thread (elements e0 + 4·fq.., positions
     // 2·pq, 2·pq+1 of the chunk); positions past tmax and elements past the
     // head clamped, never summed or stored
     const int fq = tid % (kGvElems / 4), pq = tid / (kGvElems / 4);
-    const float *vbase = vals + (int64_t)g * hs + min(e0 + 4 * fq, hs - 4);
+    const float *vbase = vals + gr.cache0 + (int64_t)g * hs + min(e0 + 4 * fq, hs - 4);
     float4 v0, v1;
     auto load_tile = [&](int c0) {
         v0 = *reinterpret_cast<const float4 *>(vbase + (int64_t)min(c0 + 2 * pq, tmax - 1) * kv_dim);
@@ -250,15 +267,18 @@ __global__ __launch_bounds__(kGvThreads) void att_values_group_kernel(const floa
     }
 }
 
+// Positions a batch's furthest token attends to, and its token groups.
+static int batch_positions(const AttBatch &bt) { return bt.groups ? bt.max_pos : bt.pos0 + bt.tokens; }
+static int batch_groups(const AttBatch &bt) { return bt.groups ? bt.ngroups : (bt.tokens + kGrpTok - 1) / kGrpTok; }
+
 bool att_group_fits(const AttBatch &bt, int hs, int kv_dim) {
-    // (consecutive positions of one sequence only)
-    return !bt.pos && bt.pos0 + bt.tokens <= kGrpMaxT && hs % 32 == 0 && kv_dim % 4 == 0;
+    // (runs of one sequence's consecutive positions only)
+    return (!bt.pos || bt.groups) && batch_positions(bt) <= kGrpMaxT && hs % 32 == 0 && kv_dim % 4 == 0;
 }
 
 void launch_att_scores_group(const float *q, const float *keys, float *att, int32_t att_stride, const AttBatch &bt,
                              int heads, int kv_heads, int kv_dim, float inv_sqrt, hipStream_t s) {
-    const int npos = bt.pos0 + bt.tokens;
-    const dim3 grid(heads, (npos + kScTile - 1) / kScTile, (bt.tokens + kGrpTok - 1) / kGrpTok);
+    const dim3 grid(heads, (batch_positions(bt) + kScTile - 1) / kScTile, batch_groups(bt));
     RK_LAUNCH(att_scores_group_kernel, grid, dim3(256), 0, s, q, keys, att, att_stride, bt, heads / kv_heads, kv_dim,
               inv_sqrt);
 }
@@ -273,10 +293,10 @@ static void launch_values_sl(const float *att, int32_t att_stride, const float *
         (void)hipFuncSetAttribute((const void *)att_values_group_kernel<SL>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kMaxLdsBytes - 12288));
     });
-    const int tmax = bt.pos0 + bt.tokens;
+    const int tmax = batch_positions(bt);
     const int apitch = ((tmax + 3) & ~3) + 4;
     const size_t lds = ((size_t)kGrpTok * apitch + 2 * kGvElems * kGvPitch) * 4;
-    const dim3 grid(heads, (hs + kGvElems - 1) / kGvElems, (bt.tokens + kGrpTok - 1) / kGrpTok);
+    const dim3 grid(heads, (hs + kGvElems - 1) / kGvElems, batch_groups(bt));
     RK_LAUNCH(att_values_group_kernel<SL>, grid, dim3(kGvThreads), lds, s, att, att_stride, vals, out, bt,
               heads / kv_heads, hs, kv_dim, apitch, qx, xs, xsum);
 }
@@ -288,7 +308,7 @@ void launch_att_values_group(const float *att, int32_t att_stride, const float *
     // unless that leaves fewer workgroups than the device has CUs (a short
     // batch; cu 0: the MI355X's 256): then one slice a workgroup, four
     // times the workgroups
-    const int64_t wgs4 = (int64_t)heads * ((hs + 127) / 128) * ((bt.tokens + kGrpTok - 1) / kGrpTok);
+    const int64_t wgs4 = (int64_t)heads * ((hs + 127) / 128) * batch_groups(bt);
     if (wgs4 >= (cu > 0 ? cu : 256))
         launch_values_sl<4>(att, att_stride, vals, out, bt, heads, kv_heads, hs, kv_dim, qx, xs, xsum, s);
     else

@@ -121,13 +121,28 @@ bool stream_has(int fmt, int pro, int epi, int cols);
 // floats into the q, scores and output buffers. Used when ctl is null.
 // Independent sequences: with `pos` set, token z is sequence z, at position
 // pos[z] (device memory), attending to its own cache, cache_stride floats
-// after sequence z-1's.
+// after sequence z-1's. Several sequences' prompts: token z at pos[z] of
+// sequence seq[z], each sequence's tokens of the batch consecutive, and
+// `groups` the runs of up to 16 of one sequence that a workgroup takes.
+constexpr int kAttGroupTok = 16;
+struct AttGroup {
+    int32_t row0, n;   // tokens row0 .. row0 + n - 1 of the batch
+    int32_t pos0, seq; // row0's position, its sequence
+};
 struct AttBatch {
     int32_t pos0 = 0, tokens = 1;
     int64_t q_stride = 0, att_stride = 0, out_stride = 0;
     const int32_t *pos = nullptr;
     int64_t cache_stride = 0;
+    const int32_t *seq = nullptr;
+    const AttGroup *groups = nullptr;  // device memory
+    int32_t ngroups = 0, max_pos = 0;  // positions the furthest token attends to
 };
+
+// Floats from the first sequence's cache to token z's.
+__device__ __forceinline__ int64_t att_cache(const AttBatch &bt, int z) {
+    return (int64_t)(bt.seq ? bt.seq[z] : z) * bt.cache_stride;
+}
 
 // Position of token z of an attention launch: the stage's (ctl), the
 // sequence's own (bt.pos), or z after the batch's first.
@@ -186,11 +201,13 @@ bool launch_att_values_wo(const float *att, int32_t att_stride, const float *val
                           unsigned long long *sync, hipStream_t s, const QknIn *qk = nullptr);
 // QK-norm (Qwen3) and RoPE of raw q and k heads, k and v into the caches, at
 // the position in ctl (or, ctl null, for `tokens` rows at pos0, pos0+1, ...;
-// or, seq_pos set, row z at seq_pos[z] in caches cache_stride floats apart).
+// or, seq_pos set, row z at seq_pos[z] in the caches of sequence z, or
+// seq[z], cache_stride floats apart).
 void launch_qknorm_rope(float *q, const float *k, const float *v, const float *q_norm, const float *k_norm,
                         float recip_hs, float eps, const float *cos_t, const float *sin_t, const int32_t *ctl,
                         int32_t pos0, int tokens, float *kcache, float *vcache, int heads, int kv_heads, int hs,
-                        hipStream_t s, const int32_t *seq_pos = nullptr, int64_t cache_stride = 0);
+                        hipStream_t s, const int32_t *seq_pos = nullptr, int64_t cache_stride = 0,
+                        const int32_t *seq = nullptr);
 // x = the embedding row of tokens[ctl[kCtlPos]] (Q8_0 or Q4_0 table), and
 // RMSNorm(x) with norm_w quantized into qx/xs/xsum (one workgroup;
 // dim <= kMaxNormCols).
@@ -199,10 +216,11 @@ void launch_embed_norm(const uint8_t *w, const float *scales, bool q4, const int
                        int32_t *xsum, hipStream_t s);
 // Embedding rows of tokens[pos0..pos0+n) (Q8_0 or Q4_0 table) into x
 // [n][dim], as embed_norm gives them one position at a time; with seq_pos,
-// row z is sequence z's token at its position, tokens[z·tok_stride +
-// seq_pos[z]].
+// row z is sequence z's (seq set: seq[z]'s) token at its position,
+// tokens[z·tok_stride + seq_pos[z]].
 void launch_embed_rows(const uint8_t *w, const float *scales, bool q4, const int32_t *tokens, int32_t pos0, int n,
-                       int dim, float *x, hipStream_t s, int64_t tok_stride = 0, const int32_t *seq_pos = nullptr);
+                       int dim, float *x, hipStream_t s, int64_t tok_stride = 0, const int32_t *seq_pos = nullptr,
+                       const int32_t *seq = nullptr);
 // Independent sequences' greedy step: the argmax of each of `seqs` logits
 // rows ([seqs][vocab]) becomes that sequence's token at pos[z]+1 (past its
 // prompt), and pos[z] advances.

@@ -598,7 +598,7 @@ __global__ __launch_bounds__(256) void att_scores_kernel(const float *q, const f
     const int T = att_position(ctl, bt, z) + 1;
     q += (int64_t)z * bt.q_stride;
     att += (int64_t)z * bt.att_stride;
-    keys += (int64_t)z * bt.cache_stride;
+    keys += att_cache(bt, z);
     const int t0 = blockIdx.y * kScoreTile;
     if (t0 >= T) return;
     const int h = blockIdx.x, g = h / kv_mul;
@@ -732,8 +732,8 @@ __global__ __launch_bounds__(256) void att_scores_qkn_kernel(const float *q_raw,
     k_raw += (int64_t)z * kv_dim;
     v_raw += (int64_t)z * kv_dim;
     att += (int64_t)z * bt.att_stride;
-    keys += (int64_t)z * bt.cache_stride;
-    vals += (int64_t)z * bt.cache_stride;
+    keys += att_cache(bt, z);
+    vals += att_cache(bt, z);
     const int h = blockIdx.x, g = h / kv_mul;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const bool here = pos < t0 + kScoreTile;  // the tile holds the position
@@ -809,7 +809,7 @@ bool launch_att_scores_qkn(const float *q_raw, const float *k_raw, const float *
                            float *keys, float *vals, float *att, int32_t att_stride, const int32_t *ctl,
                            const AttBatch &bt, int ctx, int heads, int kv_heads, int hs, int kv_dim, float inv_sqrt,
                            hipStream_t s) {
-    if (!ctl && !bt.pos) return false;  // a prompt's batch: the grouped scores, after the norm launch
+    if (!ctl && (!bt.pos || bt.seq)) return false;  // a prompt's batch: the grouped scores, after the norm launch
     if (hs % 8 != 0 || hs > kQknMaxHs || kv_dim % 4 != 0 || kv_dim != kv_heads * hs) return false;
     const dim3 grid(heads, (ctx + kScoreTile - 1) / kScoreTile, ctl ? 1 : bt.tokens);
     if (hs == 128)
@@ -876,7 +876,7 @@ __device__ __forceinline__ void att_values_body(const float *att, int32_t att_st
     const int T = att_position(ctl, bt, z) + 1;
     att += (int64_t)z * bt.att_stride;
     out += (int64_t)z * bt.out_stride;
-    vals += (int64_t)z * bt.cache_stride;
+    vals += att_cache(bt, z);
     if (qx) {
         qx += (int64_t)z * bt.out_stride;
         xs += (int64_t)z * (bt.out_stride >> 5);
@@ -1205,7 +1205,7 @@ __device__ __forceinline__ void att_values_reg_body(const float *att, int32_t at
     const int nch = (T + kVrChunk - 1) / kVrChunk;
     att += (int64_t)z * bt.att_stride;
     out += (int64_t)z * bt.out_stride;
-    vals += (int64_t)z * bt.cache_stride;
+    vals += att_cache(bt, z);
     if (qx) {
         qx += (int64_t)z * bt.out_stride;
         xs += (int64_t)z * (bt.out_stride >> 5);
@@ -1629,15 +1629,16 @@ __global__ __launch_bounds__(64) void qknorm_rope_kernel(float *q, const float *
                                                          const float *q_norm, const float *k_norm, float recip_hs,
                                                          float eps, const float *cos_t, const float *sin_t,
                                                          const int32_t *ctl, int32_t pos0, const int32_t *seq_pos,
-                                                         int64_t cache_stride, float *kcache, float *vcache,
-                                                         int heads, int hs, int kv_dim) {
+                                                         int64_t cache_stride, const int32_t *seq, float *kcache,
+                                                         float *vcache, int heads, int hs, int kv_dim) {
     // a batch: token blockIdx.y at pos0 + blockIdx.y (or, independent
-    // sequences, at seq_pos[blockIdx.y] in its own caches), rows
+    // sequences, at seq_pos[blockIdx.y] in its sequence's caches), rows
     // [tokens][heads·hs] and [tokens][kv_dim]
     const int z = blockIdx.y;
     const int pos = ctl ? ctl[kCtlPos] : seq_pos ? seq_pos[z] : pos0 + z;
-    kcache += (int64_t)z * cache_stride;
-    vcache += (int64_t)z * cache_stride;
+    const int64_t cache0 = (int64_t)(seq ? seq[z] : z) * cache_stride;
+    kcache += cache0;
+    vcache += cache0;
     q += (int64_t)z * heads * hs;
     k += (int64_t)z * kv_dim;
     v += (int64_t)z * kv_dim;
@@ -1657,10 +1658,10 @@ __global__ __launch_bounds__(64) void qknorm_rope_kernel(float *q, const float *
 void launch_qknorm_rope(float *q, const float *k, const float *v, const float *q_norm, const float *k_norm,
                         float recip_hs, float eps, const float *cos_t, const float *sin_t, const int32_t *ctl,
                         int32_t pos0, int tokens, float *kcache, float *vcache, int heads, int kv_heads, int hs,
-                        hipStream_t s, const int32_t *seq_pos, int64_t cache_stride) {
+                        hipStream_t s, const int32_t *seq_pos, int64_t cache_stride, const int32_t *seq) {
     RK_LAUNCH(qknorm_rope_kernel, dim3(heads + kv_heads, ctl ? 1 : tokens), dim3(64), 0, s, q, k, v,
-              q_norm, k_norm, recip_hs, eps, cos_t, sin_t, ctl, pos0, seq_pos, cache_stride, kcache, vcache, heads,
-              hs, kv_heads * hs);
+              q_norm, k_norm, recip_hs, eps, cos_t, sin_t, ctl, pos0, seq_pos, cache_stride, seq, kcache, vcache,
+              heads, hs, kv_heads * hs);
 }
 
 // Embedding row of the token at the position (internal/llm/model.go:216-231
@@ -1719,11 +1720,12 @@ void launch_embed_norm(const uint8_t *w, const float *scales, bool q4, const int
 // thread.
 __global__ __launch_bounds__(256) void embed_rows_kernel(const uint8_t *w, const float *scales, int q4,
                                                          const int32_t *tokens, int32_t pos0, int dim, float *x,
-                                                         int64_t tok_stride, const int32_t *seq_pos) {
+                                                         int64_t tok_stride, const int32_t *seq_pos,
+                                                         const int32_t *seq) {
     // row z: tokens[pos0 + z], or (independent sequences) sequence z's token
     // at its position, tokens[z·tok_stride + seq_pos[z]]
     const int z = blockIdx.x;
-    const int64_t tok = seq_pos ? tokens[(int64_t)z * tok_stride + seq_pos[z]] : tokens[pos0 + z];
+    const int64_t tok = seq_pos ? tokens[(int64_t)(seq ? seq[z] : z) * tok_stride + seq_pos[z]] : tokens[pos0 + z];
     const int nb = dim >> 5, ng = dim >> 2;
     float *xr = x + (int64_t)blockIdx.x * dim;
     for (int g = threadIdx.x; g < ng; g += 256) {
@@ -1743,9 +1745,9 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const uint8_t *w, const
 }
 
 void launch_embed_rows(const uint8_t *w, const float *scales, bool q4, const int32_t *tokens, int32_t pos0, int n,
-                       int dim, float *x, hipStream_t s, int64_t tok_stride, const int32_t *seq_pos) {
+                       int dim, float *x, hipStream_t s, int64_t tok_stride, const int32_t *seq_pos, const int32_t *seq) {
     RK_LAUNCH(embed_rows_kernel, dim3(n), dim3(256), 0, s, w, scales, q4 ? 1 : 0, tokens, pos0, dim, x, tok_stride,
-              seq_pos);
+              seq_pos, seq);
 }
 
 __global__ __launch_bounds__(kNormThreads) void norm_quant_kernel(const float *x, int n, const float *norm_w,

@@ -334,7 +334,7 @@ __global__ __launch_bounds__(kMmThreads) void mm_kernel(MmArgs a) {
             const int gb = row0 + rb(ti) + 4 * lq;  // the lane's first row
             if (EPI == kEpQKV) {
                 const int pos = a.seq_pos ? a.seq_pos[t] : a.pos0 + t, half = a.hs >> 1;
-                const int64_t cache0 = (int64_t)t * a.cache_stride;  // token t's sequence's caches
+                const int64_t cache0 = (int64_t)(a.seq ? a.seq[t] : t) * a.cache_stride;  // its sequence's caches
 #pragma unroll
                 for (int pr = 0; pr < 2; pr++) {
                     const int g0 = gb + 2 * pr;  // an even row: a rotary pair with g0 + 1

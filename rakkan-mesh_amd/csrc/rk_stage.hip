@@ -78,6 +78,7 @@ struct rk_stage {
     int64_t bbytes = 0;
     float *bx = nullptr, *bq = nullptr, *bk = nullptr, *bv = nullptr, *batt = nullptr, *batt_out = nullptr;
     rk::QScratch bqa{}, bqb{};
+    int32_t *btok = nullptr;  // several sequences' prompts: positions, sequences, groups (AttBatch)
     // Independent sequences (rk_stage_seqs_*): each has its own caches
     // (sequence z's at z·ctx·kv_dim in every layer's), position, prompt
     // length and tokens [ctx+1] on the device; the host keeps a copy of the
@@ -209,7 +210,7 @@ static bool enqueue_attention(rk_stage *s, hipStream_t st, const float *q, float
             ProfScope p(d, st, "qknorm_rope");
             launch_qknorm_rope(const_cast<float *>(q), qk->k, qk->v, qk->q_norm, qk->k_norm, c.recip_head, c.norm_eps,
                                s->cos_t, s->sin_t, ctl, bt.pos0, bt.tokens, keys, vals, c.heads, c.kv_heads, s->hs, st,
-                               bt.pos, bt.cache_stride);
+                               bt.pos, bt.cache_stride, bt.seq);
         }
     }
     if (!scored) {
@@ -454,10 +455,15 @@ static int batch_cap(const rk_stage_config &c, int seqs) {
 // one sequence whose caches start cache0 floats into each layer's (a
 // prompt), or one token per sequence, token z at seq_pos[z] in caches
 // cache_stride floats apart (the sequences' decode step).
+// Or (seq set) tokens of several sequences' prompts, token t at seq_pos[t]
+// of sequence seq[t], in the groups of AttBatch.
 struct BatchPos {
     int32_t pos0 = 0;
     const int32_t *seq_pos = nullptr;
     int64_t cache0 = 0, cache_stride = 0;
+    const int32_t *seq = nullptr;
+    const AttGroup *groups = nullptr;
+    int32_t ngroups = 0, max_pos = 0;
 };
 
 static int batch_alloc(rk_stage *s) {
@@ -474,6 +480,9 @@ static int batch_alloc(rk_stage *s) {
     take((void **)&s->bv, 4 * B * s->kvdim);
     take((void **)&s->batt, 4 * B * c.heads * c.ctx);
     take((void **)&s->batt_out, 4 * B * s->qdim);
+    // several sequences' prompts: each token's position and sequence, and the
+    // attention's groups (one more a sequence than whole ones)
+    if (s->seqs > 1) take((void **)&s->btok, (8 + sizeof(AttGroup)) * B + 16);
     for (QScratch *q : {&s->bqa, &s->bqb}) {
         take((void **)&q->qx, B * widest);
         take((void **)&q->xs, 4 * B * (widest / 32));
@@ -550,6 +559,7 @@ static int enqueue_layer_batch(rk_stage *s, int li, hipStream_t st, int n, const
             a.pos0 = bp.pos0;
             a.seq_pos = bp.seq_pos;
             a.cache_stride = bp.cache_stride;
+            a.seq = bp.seq;
             a.hs = s->hs;
             a.qdim = s->qdim;
             a.kvdim = s->kvdim;
@@ -576,6 +586,10 @@ static int enqueue_layer_batch(rk_stage *s, int li, hipStream_t st, int n, const
     bt.out_stride = s->qdim;
     bt.pos = bp.seq_pos;
     bt.cache_stride = bp.cache_stride;
+    bt.seq = bp.seq;
+    bt.groups = bp.groups;
+    bt.ngroups = bp.ngroups;
+    bt.max_pos = bp.max_pos;
     // the attention output comes quantized when its Q8 blocks fall within
     // heads; else it is quantized by a launch of its own
     const bool att_q = s->hs % 32 == 0;
@@ -1154,9 +1168,63 @@ int rk_stage_seqs_start(rk_stage *s, const int32_t *prompts, const int32_t *lens
     HIP_TRY(d, hipMemcpyAsync(s->seq_pos, h + S * (ctx + 1), (size_t)4 * S, hipMemcpyHostToDevice, st), "positions");
     HIP_TRY(d, hipMemcpyAsync(s->seq_prompt, h + S * (ctx + 1) + S, (size_t)4 * S, hipMemcpyHostToDevice, st),
             "prompt lengths");
-    // every prompt position but the last: each sequence's batched prefill
-    // into its own caches (the same bits as one position at a time)
-    for (int z = 0; z < S; z++) {
+    // every prompt position but the last: the batched prefill, each token
+    // into its own sequence's caches (the same bits as one position at a
+    // time). The sequences' prompts share batches where the attention takes
+    // runs of several sequences, so a batch's products read the weights once
+    // for all of them; else each sequence's prompt goes by itself.
+    AttBatch probe;
+    probe.max_pos = *std::max_element(lens, lens + S) - 1;
+    probe.groups = reinterpret_cast<const AttGroup *>(s->btok);
+    std::vector<std::vector<int32_t>> held;  // uploaded host rows, kept until the stream has them
+    if (S > 1 && att_group_fits(probe, s->hs, s->kvdim)) {
+        int z = 0, at = 0;  // the next token: sequence z's position at
+        for (;;) {
+            const int B = s->bcap;
+            std::vector<int32_t> pos, seq, grp;
+            int top = 0;
+            while (z < S && (int)pos.size() < B) {
+                const int left = lens[z] - 1 - at, n = std::min(left, B - (int)pos.size());
+                for (int g = 0; g < n; g += kAttGroupTok)
+                    grp.insert(grp.end(), {(int32_t)pos.size() + g, std::min(kAttGroupTok, n - g), at + g, z});
+                for (int i = 0; i < n; i++) {
+                    pos.push_back(at + i);
+                    seq.push_back(z);
+                }
+                top = std::max(top, at + n);
+                at += n;
+                if (n == left) {
+                    z++;
+                    at = 0;
+                }
+            }
+            const int n = (int)pos.size();
+            if (n == 0) break;
+            // one upload: positions, sequences, groups (no more than B: a
+            // group holds a token at least)
+            std::vector<int32_t> up(pos);
+            up.insert(up.end(), seq.begin(), seq.end());
+            const int goff = (2 * n + 3) & ~3;
+            up.resize(goff);
+            up.insert(up.end(), grp.begin(), grp.end());
+            held.push_back(std::move(up));
+            HIP_TRY(d, hipMemcpyAsync(s->btok, held.back().data(), held.back().size() * 4, hipMemcpyHostToDevice, st),
+                    "prompt positions");
+            BatchPos bp;
+            bp.seq_pos = s->btok;
+            bp.seq = s->btok + n;
+            bp.groups = reinterpret_cast<const AttGroup *>(s->btok + goff);
+            bp.ngroups = (int32_t)grp.size() / 4;
+            bp.max_pos = top;
+            bp.cache_stride = ctx * s->kvdim;
+            {
+                ProfScope p(d, st, "embed");
+                launch_embed_rows(s->embed->w, s->embed->scales, s->embed->kind == RK_Q4, s->seq_tokens, 0, n, s->c.dim,
+                                  s->bx, st, ctx + 1, bp.seq_pos, bp.seq);
+            }
+            if ((rc = enqueue_forward_batch(s, st, n, bp))) return rc;
+        }
+    } else for (int z = 0; z < S; z++) {
         for (int start = 0; start < lens[z] - 1; start += s->bcap) {
             const int n = std::min(s->bcap, lens[z] - 1 - start);
             {

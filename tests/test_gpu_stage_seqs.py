@@ -70,3 +70,23 @@ def test_dense_sequences_match_each_alone(dev, name):
         alone, _, _ = gpu_generate(dev, m, p, steps, ctx)
         assert alone == toks[z], f"{name}: sequence {z} alone"
     assert dev.used == 0
+
+
+@pytest.mark.parametrize("qk_norm,dtype", [(False, "q8_0"), (True, "q4_0")])
+def test_prompts_share_batches(dev, qk_norm, dtype):
+    """Prompts packed into batches of 256 tokens: runs of one token to
+    several attention groups, a sequence across two batches, sequences of
+    one token (none in a batch) at either end and between."""
+    c = Config(dim=96, hidden=160, layers=2, heads=2, kv_heads=1, vocab=50, seq_len=320, head_dim=128, qk_norm=qk_norm,
+               qkv_bias=not qk_norm, rope_theta=1e6, norm_eps=1e-6, dtype=dtype)
+    m = coded_model(c, seed=8, scale_lo=1e-3, scale_hi=1e-2)
+    rng = np.random.default_rng(4)
+    prompts = [[int(t) for t in rng.integers(0, c.vocab, n)] for n in (1, 200, 2, 1, 90, 17, 33, 1)]
+    steps, ctx = 2, 210
+    lg, toks = seqs_generate(dev, m, prompts, steps, ctx)
+    for z, p in enumerate(prompts):
+        want_t, want_l = oracle_generate(m, p, steps, ctx)
+        for k in range(steps):
+            same_bits(lg[k, z], want_l[k], f"sequence {z} (prompt {len(p)}), step {k}")
+        assert toks[z] == want_t, f"sequence {z} tokens"
+    assert dev.used == 0
