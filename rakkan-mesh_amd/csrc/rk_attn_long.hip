@@ -1,0 +1,255 @@
+// rk_attn_long.hip — decode attention over contexts past kAttLongCtx
+// positions (internal/llm/model.go:575-591): the same scores, softmax and
+// value sums, in the same order, as the shorter contexts' kernels.
+//
+// What bounds a long context: two chains of T dependent float32 adds, the
+// softmax's sum and then each output element's (about 8.7 cycles an add: 22
+// us each at 6000 positions). So nothing else may stand in their way:
+//  * The scores of a kv head's query heads share a workgroup, which holds 64
+//    positions' keys in registers: each key row is read once, not once a
+//    query head (6000 positions, 28 heads on 4: 13.4 -> 5.4 us).
+//  * Four waves load the values two chunks ahead and multiply one ahead, one
+//    wave only adds (the sums 25.5 us of a launch; the launch 65.9 -> 55).
+// Forming the softmax's sum in parallel (exactly: the sum as an integer on
+// its binade's grid, each thread's terms as how far they move an even and an
+// odd one, a scan, again after each thread that leaves the binade) measured
+// slower: 2.7 us a scan, and rows whose terms grow towards the last position
+// leave a binade every few threads (35-56 us against the chain's 22).
+#include <mutex>
+
+#include "rk_dev.h"
+#include "rk_fused.h"
+
+namespace rk {
+
+namespace {
+
+constexpr int kLongHs = 128;       // head size of the scores kernel
+constexpr int kLongTile = 64;      // positions a scores workgroup
+constexpr int kLongMaxMul = 16;    // query heads a kv head
+constexpr int kLongThreads = 512;  // values: waves 0-3 (0 adds), waves 4-7 load and multiply
+constexpr int kLongWaves = kLongThreads / 64;
+constexpr int kLongSlice = 32;     // elements a workgroup
+constexpr int kLongChunk = 256;    // positions a product tile
+
+}  // namespace
+
+// Scores of kLongTile positions for the query heads of one kv head (size
+// 128): thread (position tid/4, part tid%4) keeps its key's elements 8·part
+// .. +7 of each 32-element step in registers and runs the heads over them,
+// as quad_dot32 (the running sums j = 8·part .. +7, combined by DPP).
+__global__ __launch_bounds__(256) void att_scores_long_kernel(const float *q, const float *keys, float *att,
+                                                              int32_t att_stride, const int32_t *ctl, AttBatch bt,
+                                                              int kv_mul, int kv_dim, float inv_sqrt) {
+    __shared__ __align__(16) float sq[kLongMaxMul * kLongHs];
+    const int z = blockIdx.z;
+    const int T = att_position(ctl, bt, z) + 1;
+    const int t0 = blockIdx.y * kLongTile;
+    if (t0 >= T) return;
+    const int g = blockIdx.x, h0 = g * kv_mul;
+    const int part = threadIdx.x & 3, t = t0 + (threadIdx.x >> 2);
+    const float *kt = keys + att_cache(bt, z) + (int64_t)min(t, T - 1) * kv_dim + (int64_t)g * kLongHs + 8 * part;
+    float4 k0[kLongHs / 32], k1[kLongHs / 32];
+#pragma unroll
+    for (int st = 0; st < kLongHs / 32; st++) {
+        k0[st] = *reinterpret_cast<const float4 *>(kt + 32 * st);
+        k1[st] = *reinterpret_cast<const float4 *>(kt + 32 * st + 4);
+    }
+    const float *qh = q + (int64_t)z * bt.q_stride + (int64_t)h0 * kLongHs;
+    for (int i = threadIdx.x; i < kv_mul * (kLongHs / 4); i += 256)
+        reinterpret_cast<float4 *>(sq)[i] = reinterpret_cast<const float4 *>(qh)[i];
+    __syncthreads();
+    att += (int64_t)z * bt.att_stride;
+    for (int m = 0; m < kv_mul; m++) {
+        float s[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) s[k] = 0.0f;
+#pragma unroll
+        for (int st = 0; st < kLongHs / 32; st++) {
+            const float *qp = sq + m * kLongHs + 32 * st + 8 * part;
+            const float4 q0 = *reinterpret_cast<const float4 *>(qp), q1 = *reinterpret_cast<const float4 *>(qp + 4);
+            s[0] += q0.x * k0[st].x;
+            s[1] += q0.y * k0[st].y;
+            s[2] += q0.z * k0[st].z;
+            s[3] += q0.w * k0[st].w;
+            s[4] += q1.x * k1[st].x;
+            s[5] += q1.y * k1[st].y;
+            s[6] += q1.z * k1[st].z;
+            s[7] += q1.w * k1[st].w;
+        }
+        float e[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float u = s[k] + dppf_x1(s[k]);
+            e[k] = u + dppf_x2(u);
+        }
+        const float dot = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+        if (part == 0 && t < T) att[(int64_t)(h0 + m) * att_stride + t] = dot * inv_sqrt;
+    }
+}
+
+// Softmax and weighted values of a 32-element slice of one head (workgroup
+// x of token y): Go max, e_t = Exp32(s_t - max), the sum, inv = Recip32(sum),
+// then out_i = Σ_t (e_t·inv)·v_t,i in t order from +0. Chunk c's products
+// stand transposed and swizzled in tile c mod 2 while wave 0 adds them; waves
+// 4-7 meanwhile write chunk c+1's from registers and request chunk c+3.
+__global__ __launch_bounds__(kLongThreads) void att_values_long_kernel(const float *att, int32_t att_stride,
+                                                                       const float *vals, float *out,
+                                                                       const int32_t *ctl, AttBatch bt, int kv_mul,
+                                                                       int hs, int kv_dim, int nsl, int ctx_pad,
+                                                                       int8_t *qx, float *xs, int32_t *xsum) {
+    extern __shared__ __align__(16) float smem[];
+    __shared__ float s_red[kLongWaves];
+    __shared__ float s_inv;
+    __shared__ __align__(16) float s_res[kLongSlice];
+    float *sa = smem;               // [ctx_pad] scores -> e_t
+    float *tiles = smem + ctx_pad;  // [2][32][kLongChunk] products, swizzled rows
+    const int z = blockIdx.y;
+    const int T = att_position(ctl, bt, z) + 1;
+    const int nch = (T + kLongChunk - 1) / kLongChunk;
+    const int h = blockIdx.x / nsl, e0 = (blockIdx.x % nsl) * kLongSlice;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int u = tid - 256, fq = u & 7, pq = u >> 3;  // waves 4-7: float4 column, position quads pq and pq + 32
+    const float *vb = vals + att_cache(bt, z) + (int64_t)(h / kv_mul) * hs + e0 + 4 * fq;
+    float4 va[2][4], vc[2][4];  // even and odd chunks on their way: [quad][position in it]
+    // positions past T - 1 load T - 1's values (their products are never summed)
+    auto load = [&](float4 (&v)[2][4], int c) {
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                v[q][j] = *reinterpret_cast<const float4 *>(
+                    vb + (int64_t)min(c * kLongChunk + 4 * (pq + 32 * q) + j, T - 1) * kv_dim);
+    };
+    if (wave >= 4) {
+        load(va, 0);
+        load(vc, 1);
+    }
+    // the head's scores, eight in flight a thread
+    const float *ah = att + (int64_t)z * bt.att_stride + (int64_t)h * att_stride;
+    float m = ah[0];
+    for (int t0 = 0; t0 < T; t0 += 8 * kLongThreads) {
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = ah[min(t0 + tid + k * kLongThreads, T - 1)];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int t = t0 + tid + k * kLongThreads;
+            if (t < T) {
+                sa[t] = v[k];
+                m = gomax(m, v[k]);
+            }
+        }
+    }
+    m = wave_gomax(m);
+    if (lane == 0) s_red[wave] = m;
+    __syncthreads();
+    m = s_red[0];
+#pragma unroll
+    for (int w = 1; w < kLongWaves; w++) m = gomax(m, s_red[w]);
+    for (int t = tid; t < T; t += kLongThreads) sa[t] = exp32(sa[t] - m);
+    __syncthreads();
+    if (tid == 0) s_inv = recip32(lds_chain_sum(sa, T, 0.0f));
+    __syncthreads();
+    const float inv = s_inv;
+
+    auto products = [&](const float4 (&v)[2][4], int c) {
+        float *tile = tiles + (c & 1) * (kLongSlice * kLongChunk);
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const int qd = pq + 32 * q;  // the quad within the chunk
+            const float4 e4 = *reinterpret_cast<const float4 *>(sa + min(c * kLongChunk + 4 * qd, ctx_pad - 4));
+            const float4 a4 = make_float4(e4.x * inv, e4.y * inv, e4.z * inv, e4.w * inv);
+            const float4 p[4] = {make_float4(a4.x * v[q][0].x, a4.y * v[q][1].x, a4.z * v[q][2].x, a4.w * v[q][3].x),
+                                 make_float4(a4.x * v[q][0].y, a4.y * v[q][1].y, a4.z * v[q][2].y, a4.w * v[q][3].y),
+                                 make_float4(a4.x * v[q][0].z, a4.y * v[q][1].z, a4.z * v[q][2].z, a4.w * v[q][3].z),
+                                 make_float4(a4.x * v[q][0].w, a4.y * v[q][1].w, a4.z * v[q][2].w, a4.w * v[q][3].w)};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int i = 4 * fq + j;
+                reinterpret_cast<float4 *>(tile + i * kLongChunk)[qd ^ vr_swz(i)] = p[j];
+            }
+        }
+    };
+    float acc = 0.0f;
+    auto sums = [&](int c) {
+        if (lane < kLongSlice)
+            acc = swz_chain_sum(tiles + (c & 1) * (kLongSlice * kLongChunk) + lane * kLongChunk,
+                                min(kLongChunk, T - c * kLongChunk), vr_swz(lane), acc);
+    };
+    if (wave >= 4) {
+        products(va, 0);
+        load(va, 2);
+    }
+    __syncthreads();
+    for (int c = 0; c < nch; c += 2) {
+        if (wave == 0) {
+            sums(c);
+        } else if (wave >= 4) {  // (a chunk past the last: products that nothing reads)
+            products(vc, c + 1);
+            load(vc, c + 3);
+        }
+        __syncthreads();
+        if (wave == 0) {
+            if (c + 1 < nch) sums(c + 1);
+        } else if (wave >= 4) {
+            products(va, c + 2);
+            load(va, c + 4);
+        }
+        __syncthreads();
+    }
+    if (wave != 0) return;
+    const int64_t base = (int64_t)z * bt.out_stride + (int64_t)h * hs + e0;
+    if (lane < kLongSlice) out[base + lane] = acc;
+    if (qx) {
+        // the slice is one Q8_0 block of the next input: lanes 0-7 take
+        // four values each
+        if (lane < kLongSlice) s_res[lane] = acc;
+        const float4 v4 = reinterpret_cast<const float4 *>(s_res)[min(lane, 7)];
+        float d;
+        int cs;
+        const uint32_t pk = quantize_group(v4.x, v4.y, v4.z, v4.w, d, cs);
+        if (lane < 8) {
+            reinterpret_cast<uint32_t *>(qx + base)[lane] = pk;
+            if (lane == 0) {
+                xs[base >> 5] = d;
+                xsum[base >> 5] = cs;
+            }
+        }
+    }
+}
+
+bool launch_att_scores_long(const float *q, const float *keys, float *att, int32_t att_stride, const int32_t *ctl,
+                            const AttBatch &bt, int ctx, int heads, int kv_heads, int hs, int kv_dim, float inv_sqrt,
+                            hipStream_t s) {
+    const int kv_mul = heads / kv_heads;
+    if (ctx <= kAttLongCtx || hs != kLongHs || kv_mul < 2 || kv_mul > kLongMaxMul || kv_dim % 4 != 0 ||
+        bt.q_stride % 4 != 0 || ((reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(q)) & 15) != 0 ||
+        bt.cache_stride % 4 != 0)
+        return false;
+    const int npos = ctl || bt.pos ? ctx : bt.pos0 + bt.tokens;
+    const dim3 grid(kv_heads, (npos + kLongTile - 1) / kLongTile, ctl ? 1 : bt.tokens);
+    RK_LAUNCH(att_scores_long_kernel, grid, dim3(256), 0, s, q, keys, att, att_stride, ctl, bt, kv_mul, kv_dim, inv_sqrt);
+    return true;
+}
+
+bool launch_att_values_long(const float *att, int32_t att_stride, const float *vals, float *out, const int32_t *ctl,
+                            const AttBatch &bt, int ctx, int heads, int kv_heads, int hs, int kv_dim, int8_t *qx,
+                            float *xs, int32_t *xsum, hipStream_t s) {
+    const int ctx_pad = (ctx + 3) & ~3;
+    const size_t lds = ((size_t)ctx_pad + 2 * kLongSlice * kLongChunk) * 4;
+    if (ctx <= kAttLongCtx || hs % kLongSlice != 0 || kv_dim % 4 != 0 || bt.cache_stride % 4 != 0 ||
+        (reinterpret_cast<uintptr_t>(vals) & 15) != 0 || lds > kMaxLdsBytes - 2048)
+        return false;
+    static std::once_flag once;
+    std::call_once(once, [] {
+        (void)hipFuncSetAttribute((const void *)att_values_long_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)(kMaxLdsBytes - 2048));
+    });
+    const int nsl = hs / kLongSlice;
+    RK_LAUNCH(att_values_long_kernel, dim3(heads * nsl, ctl ? 1 : bt.tokens), dim3(kLongThreads), lds, s, att,
+              att_stride, vals, out, ctl, bt, heads / kv_heads, hs, kv_dim, nsl, ctx_pad, qx, xs, xsum);
+    return true;
+}
+
+}  // namespace rk

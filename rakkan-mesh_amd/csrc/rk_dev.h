@@ -160,6 +160,57 @@ __device__ __forceinline__ float lds_chain_sum(const float *p, int n, float acc)
     return acc;
 }
 
+// Swizzled rows: logical float4 q of row i sits at q ^ vr_swz(i), so eight
+// lanes writing eight rows 4 apart and eight lanes reading eight consecutive
+// rows both touch 32 distinct banks.
+__device__ __forceinline__ int vr_swz(int i) { return ((i >> 2) ^ ((i & 3) << 1)) & 7; }
+
+// acc + row[0] + ... + row[n-1] in order for a tile row with swizzle key
+// `key` (logical float4 q at q ^ key), n <= kVrChunk: batches of 32 values,
+// the next batch's reads in flight during the current batch's additions.
+__device__ __forceinline__ void swz_load_batch(float4 (&b)[kChainBatch], const float4 *q, int key) {
+#pragma unroll
+    for (int k = 0; k < kChainBatch; k++) b[k] = q[k ^ key];
+}
+
+__device__ __forceinline__ float swz_chain_sum(const float *row, int n, int key, float acc) {
+    const float4 *q = reinterpret_cast<const float4 *>(row);
+    const int nb = n >> 5;
+    if (nb > 0) {
+        float4 a[kChainBatch], b[kChainBatch];
+        swz_load_batch(a, q, key);
+        int k = 1;
+        for (; k + 1 < nb; k += 2) {
+            swz_load_batch(b, q + k * kChainBatch, key);
+            __builtin_amdgcn_sched_barrier(0);
+            acc = add_batch(a, acc);
+            __builtin_amdgcn_sched_barrier(0);
+            swz_load_batch(a, q + (k + 1) * kChainBatch, key);
+            __builtin_amdgcn_sched_barrier(0);
+            acc = add_batch(b, acc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (k < nb) {
+            swz_load_batch(b, q + k * kChainBatch, key);
+            __builtin_amdgcn_sched_barrier(0);
+            acc = add_batch(a, acc);
+            __builtin_amdgcn_sched_barrier(0);
+            acc = add_batch(b, acc);
+        } else {
+            acc = add_batch(a, acc);
+        }
+    }
+    for (int t = nb * 32; t < n; t += 4) {  // the last partial batch, a float4 at a time
+        const int l = t >> 2;
+        const float4 v = q[l ^ key];
+        acc += v.x;
+        if (t + 1 < n) acc += v.y;
+        if (t + 2 < n) acc += v.z;
+        if (t + 3 < n) acc += v.w;
+    }
+    return acc;
+}
+
 // Dot32's running sum of lane j (< 32) for x·x: x_i·x_i for i = j, j+32,
 // ... in order, from LDS holding x transposed (xt[j·pitch + m] = x_{j+32m},
 // pitch a multiple of 4, m < steps), in fixed-size straight-line pieces.

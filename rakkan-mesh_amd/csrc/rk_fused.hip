@@ -636,6 +636,7 @@ void launch_att_scores(const float *q, const float *keys, float *att, int32_t at
         launch_att_scores_group(q, keys, att, att_stride, bt, heads, kv_heads, kv_dim, inv_sqrt, s);
         return;
     }
+    if (launch_att_scores_long(q, keys, att, att_stride, ctl, bt, ctx, heads, kv_heads, hs, kv_dim, inv_sqrt, s)) return;
     // decode and independent sequences: positions up to ctx (tiles past a
     // token's position exit); a batch: up to its last token's
     const int npos = ctl || bt.pos ? ctx : bt.pos0 + bt.tokens;
@@ -1138,54 +1139,6 @@ constexpr int kVrChunk = 256;
 constexpr int kVrMaxChunks = 4;
 constexpr int kVrMaxCtx = kVrChunk * kVrMaxChunks;
 
-__device__ __forceinline__ int vr_swz(int i) { return ((i >> 2) ^ ((i & 3) << 1)) & 7; }
-
-// acc + row[0] + ... + row[n-1] in order for a tile row with swizzle key
-// `key` (logical float4 q at q ^ key), n <= kVrChunk: batches of 32 values,
-// the next batch's reads in flight during the current batch's additions.
-__device__ __forceinline__ void swz_load_batch(float4 (&b)[kChainBatch], const float4 *q, int key) {
-#pragma unroll
-    for (int k = 0; k < kChainBatch; k++) b[k] = q[k ^ key];
-}
-
-__device__ __forceinline__ float swz_chain_sum(const float *row, int n, int key, float acc) {
-    const float4 *q = reinterpret_cast<const float4 *>(row);
-    const int nb = n >> 5;
-    if (nb > 0) {
-        float4 a[kChainBatch], b[kChainBatch];
-        swz_load_batch(a, q, key);
-        int k = 1;
-        for (; k + 1 < nb; k += 2) {
-            swz_load_batch(b, q + k * kChainBatch, key);
-            __builtin_amdgcn_sched_barrier(0);
-            acc = add_batch(a, acc);
-            __builtin_amdgcn_sched_barrier(0);
-            swz_load_batch(a, q + (k + 1) * kChainBatch, key);
-            __builtin_amdgcn_sched_barrier(0);
-            acc = add_batch(b, acc);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (k < nb) {
-            swz_load_batch(b, q + k * kChainBatch, key);
-            __builtin_amdgcn_sched_barrier(0);
-            acc = add_batch(a, acc);
-            __builtin_amdgcn_sched_barrier(0);
-            acc = add_batch(b, acc);
-        } else {
-            acc = add_batch(a, acc);
-        }
-    }
-    for (int t = nb * 32; t < n; t += 4) {  // the last partial batch, a float4 at a time
-        const int l = t >> 2;
-        const float4 v = q[l ^ key];
-        acc += v.x;
-        if (t + 1 < n) acc += v.y;
-        if (t + 2 < n) acc += v.z;
-        if (t + 3 < n) acc += v.w;
-    }
-    return acc;
-}
-
 // The body of att_values_reg_kernel for workgroup bx of token z. SIG: the
 // values launch that also runs the Wo product (att_values_wo_kernel): the
 // slice's Q8_0 block is stored through to the device's coherence point and
@@ -1389,6 +1342,8 @@ void launch_att_values(const float *att, int32_t att_stride, const float *vals, 
                   (ctx + 3) & ~3, qx, xs, xsum);
         return;
     }
+    if (launch_att_values_long(att, att_stride, vals, out, ctl, bt, ctx, heads, kv_heads, hs, kv_dim, qx, xs, xsum, s))
+        return;
     if (vec)
         RK_LAUNCH((att_values_kernel<true, kValChunk>), grid, dim3(kValThreads), att_values_lds(ctx, kValChunk), s, att,
                   att_stride, vals, out, ctl, bt, heads / kv_heads, hs, kv_dim, ctx_pad, qx, xs, xsum);
