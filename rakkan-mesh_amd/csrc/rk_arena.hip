@@ -332,9 +332,10 @@ int rk_batch_quantize_fp8(rk_batch *b, int64_t in, int64_t n) {
     return launched(b, "quantize");
 }
 
-// internal/gpu/dsbatch.go:142-172 ExpertMatVecs: the inputs quantized into
-// the arena's quantize scratch (input k at k·cols codes), then one launch
-// over the slots.
+// internal/gpu/dsbatch.go:142-172 ExpertMatVecs: one launch over the slots,
+// which quantizes the inputs itself; inputs off 16 bytes, or in the words
+// from the first output to the last, are quantized into the scratch first
+// (input k at k·cols codes).
 int rk_batch_expert_matvecs(rk_batch *b, rk_matrix *m, int64_t per_expert, int64_t ids, int32_t slots, int64_t in,
                             int64_t in_stride, int32_t div, int64_t out, int64_t out_stride) {
     if (!b) return RK_ERR_ARGS;
@@ -358,19 +359,25 @@ int rk_batch_expert_matvecs(rk_batch *b, rk_matrix *m, int64_t per_expert, int64
     if (!idw) return b->err;
     for (int32_t k = 0; k < slots; k++)
         if (!span(b, out + k * out_stride, per_expert, "expert output")) return b->err;
+    for (int64_t k = 0; k < inputs; k++)
+        if (!span(b, in + k * in_stride, cols, "expert input")) return b->err;
     float *o = a->buf + out;
+    const float *x = a->buf + in;
     hipStream_t s = d->stream;
-    {
+    // (every span above lies in the arena, so neither product overflows)
+    const int64_t x_last = (inputs - 1) * in_stride, o_last = (slots - 1) * out_stride;
+    const bool floats = mx_takes_floats(x + std::min<int64_t>(x_last, 0), std::abs(x_last) + cols, in_stride,
+                                        o + std::min<int64_t>(o_last, 0), std::abs(o_last) + per_expert);
+    if (!floats) {
         ProfScope p(d, s, "act_fp8");
-        for (int64_t k = 0; k < inputs; k++) {
-            const float *x = span(b, in + k * in_stride, cols, "expert input");
-            if (!x) return b->err;
-            launch_act_fp8(x, cols, reinterpret_cast<uint8_t *>(a->qx) + k * cols, a->xs + k * (cols / 32), s);
-        }
+        for (int64_t k = 0; k < inputs; k++)
+            launch_act_fp8(x + k * in_stride, cols, reinterpret_cast<uint8_t *>(a->qx) + k * cols,
+                           a->xs + k * (cols / 32), s);
     }
     ProfScope p(d, s, "matvec_fp4_experts");
     launch_mx_experts(m->w, m->e8m0, m->rows / per_expert, per_expert, cols, reinterpret_cast<const uint32_t *>(idw),
-                      slots, div, reinterpret_cast<const uint8_t *>(a->qx), a->xs, o, out_stride, m->raw != 0, s);
+                      slots, div, reinterpret_cast<const uint8_t *>(a->qx), a->xs, floats ? x : nullptr, in_stride, o, out_stride,
+                      m->raw != 0, s);
     return launched(b, "expert products");
 }
 

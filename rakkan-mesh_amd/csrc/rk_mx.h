@@ -26,22 +26,29 @@ void launch_fp4_quant_inplace(float *x, int64_t n, bool e4m3, hipStream_t s);
 int64_t mx_fp4_scale_bytes(int64_t rows, int64_t cols);
 void mx_fp4_pack_scales(const uint8_t *e8m0, int64_t rows, int64_t cols, uint8_t *dst);
 
+// Whether a product may read its n input floats itself: they (and rows of
+// them stride apart) lie on 16 bytes and share no byte with the out_n floats
+// it writes, which other workgroups may not have read yet.
+bool mx_takes_floats(const float *x, int64_t n, int64_t stride, const float *out, int64_t out_n);
+
 // internal/num/mx.go:282-334 MatVecFP8 / MatVecFP4 of an input quantized by
 // launch_act_fp8 (codes xc, scales xs): out[r] for rows rows; w E4M3
 // [rows][cols] with E8M0 scales [ceil(rows/32)][cols/32] (fp4 = false), or
 // E2M1 packed [rows][cols/2] with E8M0 scales in mx_fp4_pack_scales's
 // layout (fp4 = true). raw leaves the sums in float32 instead of rounding
 // them to bfloat16.
+// x set: the kernel quantizes the float32 input itself (no codes or scales).
 void launch_mx_matvec(bool fp4, const uint8_t *w, const uint8_t *ws, int64_t rows, int64_t cols, const uint8_t *xc,
-                      const float *xs, float *out, bool raw, hipStream_t s);
+                      const float *xs, const float *x, float *out, bool raw, hipStream_t s);
 
 // internal/gpu/dsbatch.go:142-172 ExpertMatVecs: E2M1 experts of per_expert
 // rows stacked in w (experts of them; per_expert a multiple of 8); slot y
 // (of slots) multiplies expert ids[y] (device memory; ids not below experts
 // are skipped) by input y / div (codes xc + (y/div)·cols, scales
-// xs + (y/div)·cols/32) into out + y·out_stride.
+// xs + (y/div)·cols/32; or, x set, the float32 values x + (y/div)·x_stride)
+// into out + y·out_stride.
 void launch_mx_experts(const uint8_t *w, const uint8_t *ws, int64_t experts, int64_t per_expert, int64_t cols,
-                       const uint32_t *ids, int slots, int div, const uint8_t *xc, const float *xs, float *out,
-                       int64_t out_stride, bool raw, hipStream_t s);
+                       const uint32_t *ids, int slots, int div, const uint8_t *xc, const float *xs, const float *x,
+                       int64_t x_stride, float *out, int64_t out_stride, bool raw, hipStream_t s);
 
 }  // namespace rk

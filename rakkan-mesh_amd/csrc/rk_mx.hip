@@ -34,7 +34,12 @@
 // them in block order (a sequential float32 chain, lds_chain_sum). Rows
 // wider than the workgroup's lanes take several chunks, the chain carried
 // across them. With a slot table the grid's second dimension runs selected
-// experts (ExpertMatVecs). Also here: the in-place E4M3 / E2M1 quantizers
+// experts (ExpertMatVecs). A lane quantizes its own input slice while the
+// weights are on their way (mx_quantize): a product takes 1.1-2.3 us longer
+// (32768x1280 E4M3 11.1 -> 13.4, 5120x8192 10.8 -> 12.0, six experts of
+// 2304x5120 E2M1 12.4 -> 13.5, of 5120x2304 11.8 -> 13.6) and the launch
+// before it, 3.4 us and a gap an input, goes (those two projections and three
+// expert products, ten quantized inputs: 143.6 -> 125.5 us). Also here: the in-place E4M3 / E2M1 quantizers
 // of the DeepSeek batch (ActQuantInPlace, FP4QuantInPlace).
 #include <algorithm>
 #include <mutex>
@@ -248,7 +253,7 @@ struct XSlice;
 template <int NE>
 struct XSlice<false, NE> {
     double v[NE];
-    __device__ void init(const uint32_t (&xw)[NE / 4]) {
+    __device__ void init(const uint32_t (&xw)[NE / 4], bool) {
 #pragma unroll
         for (int k = 0; k < NE / 4; k++) {
             const rk_f2 lo = __builtin_amdgcn_cvt_pk_f32_fp8(xw[k], false);
@@ -261,22 +266,73 @@ template <int NE>
 struct XSlice<true, NE> {
     rk_h2 h[NE / 2];
     uint32_t nanmask;
-    __device__ void init(const uint32_t (&xw)[NE / 4]) {
+    __device__ void init(const uint32_t (&xw)[NE / 4], bool nans) {  // nans: xw may hold NaN codes
         nanmask = 0;
 #pragma unroll
         for (int k = 0; k < NE / 4; k++) {
             uint32_t u = xw[k];
+            if (nans) {
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (((u >> (8 * j)) & 0x7f) == 0x7f) {  // NaN code: 0 here, its position kept
-                    nanmask |= 1u << (4 * k + j);
-                    u &= ~(0xffu << (8 * j));
-                }
+                for (int j = 0; j < 4; j++)
+                    if (((u >> (8 * j)) & 0x7f) == 0x7f) {  // NaN code: 0 here, its position kept
+                        nanmask |= 1u << (4 * k + j);
+                        u &= ~(0xffu << (8 * j));
+                    }
+            }
             h[2 * k] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u, 1.0f, false);
             h[2 * k + 1] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(u, 1.0f, true);
         }
     }
 };
+
+// A product's input: E4M3 codes and block scales (launch_act_fp8's), or
+// float32 values that each workgroup quantizes itself (XF); of a launch over
+// slots, input k's values at k·stride.
+struct MxIn {
+    const uint8_t *codes;
+    const float *scales;
+    const float *x;
+    int64_t stride;
+};
+
+// QuantizeActFP8 of a block whose LB lanes hold NE = 32/LB values each: the
+// lane's codes and the block's scale; true if the codes may hold NaNs. The
+// maximum is taken on the bits without the sign (infinities and NaNs above
+// every finite value). A finite block's scale is a normal power of two with
+// no |v|/s past 448·(1 + 2^-23), where the hardware's conversion (to nearest
+// even, subnormals kept) gives the codes of EncodeE4M3; a block with an
+// infinity or NaN takes the general code.
+template <int LB>
+__device__ __forceinline__ bool mx_quantize(const float4 (&xv)[8 / LB], uint32_t (&xw)[8 / LB], float &scale) {
+    uint32_t top = 0;
+#pragma unroll
+    for (int k = 0; k < 8 / LB; k++) {
+        top = max(max(top, f2u(xv[k].x) & 0x7fffffffu), f2u(xv[k].y) & 0x7fffffffu);
+        top = max(max(top, f2u(xv[k].z) & 0x7fffffffu), f2u(xv[k].w) & 0x7fffffffu);
+    }
+#pragma unroll
+    for (int o = 1; o < LB; o <<= 1) top = max(top, (uint32_t)__shfl_xor((int)top, o));
+    const float s = pow2ceil(gomax(u2f(top), kActFloor) * kInv448);
+    scale = s;
+    if (top < 0x7f800000u) {
+        const float inv = u2f(0x7f000000u - f2u(s));  // 1/s, a power of two
+#pragma unroll
+        for (int k = 0; k < 8 / LB; k++) {
+            const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(xv[k].x * inv, xv[k].y * inv, 0, false);
+            xw[k] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(xv[k].z * inv, xv[k].w * inv, lo, true);
+        }
+        return false;
+    }
+#pragma unroll
+    for (int k = 0; k < 8 / LB; k++) {
+        const float v[4] = {xv[k].x, xv[k].y, xv[k].z, xv[k].w};
+        xw[k] = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            xw[k] |= encode_e4m3(gomin(gomax(__fdiv_rn(v[j], s), -448.0f), 448.0f)) << (8 * j);
+    }
+    return true;
+}
 
 // Where a lane's loads go: G rows side by side, each lane one block of row
 // gl of each step.
@@ -405,11 +461,13 @@ __device__ __forceinline__ MxLane mx_lane(const uint8_t *w, const uint8_t *ws, i
 // rows read as long runs), RT steps. Lane group lg (LB lanes) takes block lg mod nb of row lg / nb
 // within the step; rows wider than the workgroup's lanes take chunks of cb
 // blocks (G = 1), the chains carried across them.
-template <bool FP4, bool SIDE, int LB, int RT>
+template <bool FP4, bool SIDE, int LB, int RT, bool XF>
 __global__ __launch_bounds__(512) void mx_matvec_kernel(const uint8_t *__restrict__ w, const uint8_t *__restrict__ ws,
-                                                        int64_t rows, int cols, int G, const uint8_t *__restrict__ xc,
-                                                        const float *__restrict__ xs, float *__restrict__ out,
-                                                        int raw, MxSlots S) {
+                                                        int64_t rows, int cols, int G, MxIn in,
+                                                        float *__restrict__ out, int raw, MxSlots S) {
+    const uint8_t *__restrict__ xc = in.codes;
+    const float *__restrict__ xs = in.scales;
+    const float *__restrict__ xf = in.x;
     if (S.ids) {
         // slot blockIdx.y: the expert its id names (rows experts of S.per
         // rows from w), its input, its output; ids outside the part are
@@ -421,8 +479,12 @@ __global__ __launch_bounds__(512) void mx_matvec_kernel(const uint8_t *__restric
         ws += FP4 ? (int64_t)e * S.per * nb : (int64_t)e * S.per / 32 * nb;
         rows = S.per;
         const int inp = blockIdx.y / S.div;
-        xc += (int64_t)inp * cols;
-        xs += (int64_t)inp * nb;
+        if constexpr (XF) {
+            xf += inp * in.stride;
+        } else {
+            xc += (int64_t)inp * cols;
+            xs += (int64_t)inp * nb;
+        }
         out += blockIdx.y * S.out_stride;
     }
     constexpr int NE = 32 / LB;
@@ -444,14 +506,23 @@ __global__ __launch_bounds__(512) void mx_matvec_kernel(const uint8_t *__restric
         // the input slice first (loads complete in issue order: it is then
         // ready while the weights are still on their way)
         uint32_t xw[NE / 4];
+        float4 xv[XF ? NE / 4 : 1];
+        float xsb = 0.0f;
+        if constexpr (XF) {
 #pragma unroll
-        for (int k = 0; k < NE / 4; k++) xw[k] = *reinterpret_cast<const uint32_t *>(xc + b * 32 + p * NE + 4 * k);
-        const float xsb = xs[b];
+            for (int k = 0; k < NE / 4; k++) xv[k] = *reinterpret_cast<const float4 *>(xf + b * 32 + p * NE + 4 * k);
+        } else {
+#pragma unroll
+            for (int k = 0; k < NE / 4; k++) xw[k] = *reinterpret_cast<const uint32_t *>(xc + b * 32 + p * NE + 4 * k);
+            xsb = xs[b];
+        }
         WT wv[RT];
         uint32_t wsv[RT];
         mx_load_tile<FP4, SIDE, LB, RT>(L, blockIdx.x, wv, wsv);
         XSlice<FP4, NE> x;
-        x.init(xw);
+        bool nans = true;
+        if constexpr (XF) nans = mx_quantize<LB>(xv, xw, xsb);
+        x.init(xw, nans);
         mx_tile_terms<FP4, LB, RT>(wv, wsv, x, xsb, p == 0 && live, G, g, bi, ts, terms);
         __syncthreads();
         if constexpr (SIDE) {
@@ -518,33 +589,41 @@ MxShape mx_shape(bool fp4, int nb) {
     return best;
 }
 
-template <bool FP4, bool SIDE, int LB, int RT>
-void launch_mx_t(const uint8_t *w, const uint8_t *ws, int64_t rows, int cols, const uint8_t *xc, const float *xs,
-                 float *out, bool raw, int G, int waves, const MxSlots &S, int slots, hipStream_t s) {
+template <bool FP4, bool SIDE, int LB, int RT, bool XF>
+void launch_mx_x(const uint8_t *w, const uint8_t *ws, int64_t rows, int cols, const MxIn &in, float *out, bool raw,
+                 int G, int waves, const MxSlots &S, int slots, hipStream_t s) {
     static std::once_flag once;
     std::call_once(once, [] {
-        (void)hipFuncSetAttribute((const void *)mx_matvec_kernel<FP4, SIDE, LB, RT>,
+        (void)hipFuncSetAttribute((const void *)mx_matvec_kernel<FP4, SIDE, LB, RT, XF>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     });
     const int nb = cols / 32, cb = SIDE ? nb : 64 * waves / LB;
     const size_t lds = (size_t)RT * G * term_stride(cb) * 4;
     const int64_t per = (int64_t)RT * G;
     const int64_t tiles = (rows + per - 1) / per;
-    RK_LAUNCH((mx_matvec_kernel<FP4, SIDE, LB, RT>), dim3((unsigned)tiles, (unsigned)slots), dim3((unsigned)(64 * waves)),
-              lds, s, w, ws, rows, cols, G, xc, xs, out, raw ? 1 : 0, S);
+    RK_LAUNCH((mx_matvec_kernel<FP4, SIDE, LB, RT, XF>), dim3((unsigned)tiles, (unsigned)slots), dim3((unsigned)(64 * waves)),
+              lds, s, w, ws, rows, cols, G, in, out, raw ? 1 : 0, S);
+}
+
+template <bool FP4, bool SIDE, int LB, int RT>
+void launch_mx_t(const uint8_t *w, const uint8_t *ws, int64_t rows, int cols, const MxIn &in, float *out, bool raw,
+                 int G, int waves, const MxSlots &S, int slots, hipStream_t s) {
+    if (in.x)
+        launch_mx_x<FP4, SIDE, LB, RT, true>(w, ws, rows, cols, in, out, raw, G, waves, S, slots, s);
+    else
+        launch_mx_x<FP4, SIDE, LB, RT, false>(w, ws, rows, cols, in, out, raw, G, waves, S, slots, s);
 }
 
 void launch_mx_any(bool fp4, const MxShape &sh, const uint8_t *w, const uint8_t *ws, int64_t rows, int cols,
-                   const uint8_t *xc, const float *xs, float *out, bool raw, const MxSlots &S, int slots,
-                   hipStream_t s) {
+                   const MxIn &in, float *out, bool raw, const MxSlots &S, int slots, hipStream_t s) {
     if (fp4 && sh.g > 1)
-        launch_mx_t<true, true, 1, kMxStepsFp4>(w, ws, rows, cols, xc, xs, out, raw, sh.g, sh.waves, S, slots, s);
+        launch_mx_t<true, true, 1, kMxStepsFp4>(w, ws, rows, cols, in, out, raw, sh.g, sh.waves, S, slots, s);
     else if (fp4)
-        launch_mx_t<true, false, 1, kMxStepsFp4>(w, ws, rows, cols, xc, xs, out, raw, 1, sh.waves, S, slots, s);
+        launch_mx_t<true, false, 1, kMxStepsFp4>(w, ws, rows, cols, in, out, raw, 1, sh.waves, S, slots, s);
     else if (sh.g > 1)
-        launch_mx_t<false, true, 2, kMxStepsFp8>(w, ws, rows, cols, xc, xs, out, raw, sh.g, sh.waves, S, slots, s);
+        launch_mx_t<false, true, 2, kMxStepsFp8>(w, ws, rows, cols, in, out, raw, sh.g, sh.waves, S, slots, s);
     else
-        launch_mx_t<false, false, 2, kMxStepsFp8>(w, ws, rows, cols, xc, xs, out, raw, 1, sh.waves, S, slots, s);
+        launch_mx_t<false, false, 2, kMxStepsFp8>(w, ws, rows, cols, in, out, raw, 1, sh.waves, S, slots, s);
 }
 
 }  // namespace
@@ -585,8 +664,13 @@ void launch_fp4_quant_inplace(float *x, int64_t n, bool e4m3, hipStream_t s) {
         RK_LAUNCH(fp4_quant_inplace_kernel<false>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x, n);
 }
 
+bool mx_takes_floats(const float *x, int64_t n, int64_t stride, const float *out, int64_t out_n) {
+    const uintptr_t x0 = (uintptr_t)x, x1 = x0 + 4 * (uintptr_t)n, o0 = (uintptr_t)out, o1 = o0 + 4 * (uintptr_t)out_n;
+    return x0 % 16 == 0 && stride % 4 == 0 && (x1 <= o0 || o1 <= x0);
+}
+
 void launch_mx_matvec(bool fp4, const uint8_t *w, const uint8_t *ws, int64_t rows, int64_t cols, const uint8_t *xc,
-                      const float *xs, float *out, bool raw, hipStream_t s) {
+                      const float *xs, const float *x, float *out, bool raw, hipStream_t s) {
     const MxShape sh = mx_shape(fp4, (int)(cols / 32));
     const int64_t rb = fp4 ? cols / 2 : cols, nb = cols / 32;
     // parts of at most 1 GiB of weights, whole 32-row scale blocks (and so
@@ -596,14 +680,14 @@ void launch_mx_matvec(bool fp4, const uint8_t *w, const uint8_t *ws, int64_t row
     const MxSlots none{nullptr, 0, 0, 0, 0, 1};
     for (int64_t r0 = 0; r0 < rows; r0 += per) {
         const int64_t n = std::min(per, rows - r0);
-        launch_mx_any(fp4, sh, w + r0 * rb, ws + (fp4 ? r0 * nb : r0 / 32 * nb), n, (int)cols, xc, xs, out + r0, raw,
+        launch_mx_any(fp4, sh, w + r0 * rb, ws + (fp4 ? r0 * nb : r0 / 32 * nb), n, (int)cols, MxIn{xc, xs, x, 0}, out + r0, raw,
                       none, 1, s);
     }
 }
 
 void launch_mx_experts(const uint8_t *w, const uint8_t *ws, int64_t experts, int64_t per_expert, int64_t cols,
-                       const uint32_t *ids, int slots, int div, const uint8_t *xc, const float *xs, float *out,
-                       int64_t out_stride, bool raw, hipStream_t s) {
+                       const uint32_t *ids, int slots, int div, const uint8_t *xc, const float *xs, const float *x,
+                       int64_t x_stride, float *out, int64_t out_stride, bool raw, hipStream_t s) {
     const MxShape sh = mx_shape(true, (int)(cols / 32));
     const int64_t rb = cols / 2, nb = cols / 32;
     // parts of whole experts, at most 1 GiB of weights each
@@ -611,8 +695,8 @@ void launch_mx_experts(const uint8_t *w, const uint8_t *ws, int64_t experts, int
     for (int64_t e0 = 0; e0 < experts; e0 += per) {
         const int64_t ne = std::min(per, experts - e0);
         const MxSlots S{ids, per_expert, out_stride, (int32_t)e0, (int32_t)ne, div};
-        launch_mx_any(true, sh, w + e0 * per_expert * rb, ws + e0 * per_expert * nb, per_expert, (int)cols, xc, xs, out,
-                      raw, S, slots, s);
+        launch_mx_any(true, sh, w + e0 * per_expert * rb, ws + e0 * per_expert * nb, per_expert, (int)cols,
+                      MxIn{xc, xs, x, x_stride}, out, raw, S, slots, s);
     }
 }
 

@@ -161,21 +161,30 @@ int enqueue_matvecs(rk_device *d, int32_t n, rk_matrix *const *ms, float *const 
         int rc = flush();
         if (rc) return rc;
     }
-    // E4M3 / E2M1 matrices: the input quantized once to E4M3 with block
-    // scales into the scratch (internal/gpu/batch.go:221-233 QuantizeFP8),
-    // then one launch each. (Quantizing inside the products was measured
-    // slower: every workgroup of a few rows quantizes the whole input.)
-    bool mx_quantized = false;
+    // E4M3 / E2M1 matrices, one launch each, the input quantized to E4M3 with
+    // block scales (internal/gpu/batch.go:221-233 QuantizeFP8) inside it: a
+    // lane quantizes only its own slice, by the hardware's conversion, while
+    // the weights are on their way. An input off 16 bytes, or one that a
+    // matrix's output overlaps, is quantized once into the scratch first; so
+    // is one of more than three matrices (a product takes up to 2.3 us longer
+    // for it, the launch and its gap about 7).
+    bool mx_floats = true, mx_quantized = false;
+    int mx_count = 0;
+    for (int i = 0; i < n; i++) {
+        mx_floats = mx_floats && mx_takes_floats(x, cols, 0, outs[i], ms[i]->rows);
+        mx_count += ms[i]->kind == RK_FP8 || ms[i]->kind == RK_FP4;
+    }
+    mx_floats = mx_floats && mx_count <= 3;
     for (int i = 0; i < n; i++) {
         if (ms[i]->kind != RK_FP8 && ms[i]->kind != RK_FP4) continue;
-        if (!mx_quantized) {
+        if (!mx_floats && !mx_quantized) {
             ProfScope p(d, s, "act_fp8");
             launch_act_fp8(x, cols, reinterpret_cast<uint8_t *>(q.qx), q.xs, s);
             mx_quantized = true;
         }
         ProfScope p(d, s, ms[i]->kind == RK_FP8 ? "matvec_fp8" : "matvec_fp4");
         launch_mx_matvec(ms[i]->kind == RK_FP4, ms[i]->w, ms[i]->e8m0, ms[i]->rows, cols,
-                         reinterpret_cast<const uint8_t *>(q.qx), q.xs, outs[i], ms[i]->raw != 0, s);
+                         reinterpret_cast<const uint8_t *>(q.qx), q.xs, mx_floats ? x : nullptr, outs[i], ms[i]->raw != 0, s);
     }
     // float32 / bfloat16 matrices take x as it is (internal/gpu/batch.go:
     // 263-264: no quantized input), up to three of a format a launch

@@ -569,3 +569,68 @@ def test_chunked_upload_errors(dev):
     m = dev.upload_mx_chunks(rkhip.FP4, 6, 64, [z(192)], [z(12)], align_rows=3)
     m.free()
     assert dev.used == 0
+
+
+@pytest.mark.parametrize("cols", [32, 160, 1280, 2304, 5120, 9216])
+def test_input_quantized_inside_the_product(dev, cols):
+    """Inputs at and one float32 step beside the E4M3 rounding ties, over the
+    scales' range, with block maxima at and one step past 448 times a power
+    of two: the products' bits are the CPU's (widths: one block, rows side by
+    side, one row a workgroup, several chunks a row)."""
+    rng = np.random.default_rng(cols + 1)
+    codes = e4m3_f32(np.arange(0x7F, dtype=np.uint8))  # 0 .. 448
+    ties = (codes[:-1] + codes[1:]) / 2
+    w8, s8 = random_fp8(rng, 40, cols)
+    w4 = rng.integers(0, 256, 40 * cols // 2).astype(np.uint8)
+    s4 = random_scales(rng, 40 * cols // 32)
+    m8, m4 = dev.upload_mx(rkhip.FP8, 40, cols, w8, s8), dev.upload_mx(rkhip.FP4, 40, cols, w4, s4)
+    try:
+        for _ in range(6):
+            v = rng.choice(np.concatenate([ties, codes]), cols).astype(np.float32)
+            step = rng.integers(-1, 2, cols)
+            v = np.where(step < 0, np.nextafter(v, np.float32(0)),
+                         np.where(step > 0, np.nextafter(v, np.float32(500)), v)).astype(np.float32)
+            top = np.float32(448)
+            v[::32] = rng.choice([top, np.nextafter(top, np.float32(0)), np.nextafter(top, np.float32(500))], cols // 32)
+            x = np.ldexp(v, np.repeat(rng.integers(-24, 110, cols // 32), 32)).astype(np.float32)
+            x *= rng.choice(np.array([-1, 1], np.float32), cols)
+            check_both(dev, m8, x, lambda r: oracle.matvec_fp8(w8, s8, x, 40, cols, r))
+            check_both(dev, m4, x, lambda r: oracle.matvec_fp4(w4, s4, x, 40, cols, r))
+    finally:
+        m8.free()
+        m4.free()
+
+
+def test_output_over_the_input(dev):
+    """Products and expert products whose output takes the input's place:
+    every row and slot multiplies the input as it was."""
+    rng = np.random.default_rng(31)
+    cols, P, E = 1024, 1024, 3
+    x = mx_input(rng, cols, specials=True)
+    w8, s8 = random_fp8(rng, 1000, cols)
+    w4 = rng.integers(0, 256, E * P * cols // 2).astype(np.uint8)
+    s4 = random_scales(rng, E * P * cols // 32)
+    ids = np.array([2, 0], np.uint32)
+    ms = [dev.upload_mx(rkhip.FP8, 1000, cols, w8, s8), dev.upload_mx(rkhip.FP4, E * P, cols, w4, s4)]
+    arena = dev.arena(8192, 16384)
+    arena.set_quant_scratch(6144, 7680)
+    try:
+        b = arena.begin()
+        b.write(0, x)
+        b.matvecs([ms[0], ms[0]], [0, 2048], 0)
+        got = [np.asarray(b.read(o, 1000)) for o in (0, 2048)]
+        b.write(0, x)
+        b.write(4096, ids.view(np.float32))
+        b.expert_matvecs(ms[1], P, 4096, 2, 0, 0, 0, 0, P)
+        ex = np.asarray(b.read(0, 2 * P)).reshape(2, P)
+        b.submit()
+        for g in got:
+            same_bits(g, oracle.matvec_fp8(w8, s8, x, 1000, cols), "output over the input")
+        for k, e in enumerate(ids):
+            want = oracle.matvec_fp4(w4[e * P * cols // 2:(e + 1) * P * cols // 2],
+                                     s4[e * P * cols // 32:(e + 1) * P * cols // 32], x, P, cols)
+            same_bits(ex[k], want, f"slot {k}")
+    finally:
+        arena.free()
+        for m in ms:
+            m.free()
