@@ -71,13 +71,12 @@ struct rk_device {
     int64_t used = 0;
     std::string err;
     // Scratch of the standalone products (the reference's host arena):
-    // input, its Q8 form, outputs, and pinned staging for the copies.
+    // input, its Q8 form, and pinned staging for the input and the outputs.
     float *x = nullptr;
     int8_t *qx = nullptr;
     float *xs = nullptr;
     int32_t *xsum = nullptr;
-    float *out = nullptr;
-    float *h_stage = nullptr;
+    float *h_stage = nullptr, *h_stage_d = nullptr;  // the same words, as the host and as kernels address them
     // Scratch of the batched products (rk_matmul_t*), grown on demand:
     // quantized inputs [tokens][cols] (codes; scales and code sums per block),
     // and f32 input/output for the host-buffer call.
