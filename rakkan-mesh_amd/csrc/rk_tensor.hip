@@ -43,12 +43,14 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int rk_i2 __attribute__((ext_vector_type(2)));
 
-// Tile order: workgroup ids go round the 8 XCDs, so id mod 8 picks a
-// contiguous run of tiles (along n first): an XCD's workgroups then share
-// rows of a and columns of b in its own L2. -1: past the last tile.
+// Tile order: workgroup ids (tile_grid's rows one after the other, each a
+// multiple of 8) go round the 8 XCDs, so id mod 8 picks a contiguous run of
+// tiles (along n first): an XCD's workgroups then share rows of a and columns
+// of b in its own L2. -1: past the last tile.
 __device__ __forceinline__ int64_t xcd_tile(int64_t tiles) {
-    const int64_t per = (tiles + 7) >> 3, t = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    return (blockIdx.x >> 3) < per && t < tiles ? t : -1;
+    const int64_t id = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+    const int64_t per = (tiles + 7) >> 3, t = (id & 7) * per + (id >> 3);
+    return (id >> 3) < per && t < tiles ? t : -1;
 }
 
 // ---- f32 ----
@@ -402,8 +404,12 @@ static unsigned elem_grid(int64_t n) { return (unsigned)std::min<int64_t>((n + 2
 static int64_t tiles_of(int64_t m, int64_t n, int tm, int tn) { return ((m + tm - 1) / tm) * ((n + tn - 1) / tn); }
 
 // One workgroup a tile, the count padded to whole rounds of the 8 XCDs
-// (xcd_tile). 2^31 tiles are 2^41 outputs: more than the memory.
-static dim3 tile_grid(int64_t m, int64_t n, int tm, int tn) { return dim3((unsigned)((tiles_of(m, n, tm, tn) + 7) / 8 * 8)); }
+// (xcd_tile), in rows of 2^20 workgroups: a grid dimension takes fewer than
+// 2^32 threads, 2^24 of these workgroups (2^34 float32 outputs, 64 GiB).
+static dim3 tile_grid(int64_t m, int64_t n, int tm, int tn) {
+    const int64_t ids = (tiles_of(m, n, tm, tn) + 7) / 8 * 8, row = std::min<int64_t>(ids, 1 << 20);
+    return dim3((unsigned)row, (unsigned)((ids + row - 1) / row));
+}
 
 template <int TM, int TN, int KC, int WM, int WN, int WK, bool TRANS>
 static void launch_tensor_i8_t(const int8_t *a, const int8_t *b, int32_t *c, int64_t m, int64_t k, int64_t n,

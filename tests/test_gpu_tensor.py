@@ -151,3 +151,27 @@ def test_i8_tiles(dev, m, k, n, off):
         q.submit()
         assert np.array_equal(got.view(np.int32).reshape(m, n), want)
     arena.free()
+
+
+# More tiles than one grid dimension takes (2^24 workgroups of 256 threads).
+def test_f32_more_tiles_than_a_grid_dimension(dev):
+    m = n = 1 << 17
+    rng = np.random.default_rng(17)
+    a, b = rng.normal(0, 1, (2, m)).astype(np.float32)
+    at_c = 2 * m
+    arena = dev.arena(at_c + m * n, 2 * m + 8 * n)
+    try:
+        q = arena.begin()
+        q.write(0, a)
+        q.write(m, b)
+        q.submit()
+        dev._check(rkhip.lib().rk_tensor_matmul_device(dev.h, rkhip.TENSOR_F32, 0, m, 1, n, arena.device_ptr(0),
+                                                       arena.device_ptr(m), arena.device_ptr(at_c), None))
+        rows = [0, 1, 31, 32, 65537, 100003, m - 33, m - 1]
+        q = arena.begin()
+        got = [q.read(at_c + i * n, n) for i in rows]
+        q.submit()
+        for i, g in zip(rows, got):
+            assert np.array_equal(bits(np.asarray(g)), bits(np.float32(0) + a[i] * b)), i
+    finally:
+        arena.free()
