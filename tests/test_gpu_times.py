@@ -1,0 +1,47 @@
+"""Kernel times beside each other: of the same work where a configuration
+does not add any (a longer context, a padded slice), and of less work
+against more. Each is the profiler's time of a call's launches, the least of
+several calls; the bounds leave half of the difference that the right launch
+makes."""
+import numpy as np
+import pytest
+
+import rkhip
+from oracle.model import Config
+from test_gpu_fused_stage import coded_model, make_stage, upload_layers
+
+pytestmark = pytest.mark.gpu
+
+
+def profile(dev, run):
+    """{kernel: (launches, ms)} of run()."""
+    dev.profile_start()
+    try:
+        run()
+    finally:
+        prof = dev.profile_stop()
+    return prof
+
+
+def least_ms(dev, run, kernel, calls=7):
+    return min(profile(dev, run)[kernel][1] for _ in range(calls))
+
+
+@pytest.mark.parametrize("transposed", [0, 1])
+def test_tensor_positions_past_k_cost_nothing(dev, transposed):
+    """2048 x k x 2048 float32: a slice of 8 positions against a whole one."""
+    n = 2048
+    arena = dev.arena(2 * n * 64 + n * n, 64)
+    try:
+        def run(k):
+            dev._check(rkhip.lib().rk_tensor_matmul_device(dev.h, rkhip.TENSOR_F32, transposed, n, k, n,
+                                                           arena.device_ptr(0), arena.device_ptr(64 * n),
+                                                           arena.device_ptr(128 * n), None))
+
+        ms = {k: least_ms(dev, lambda: [run(k) for _ in range(10)], "tensor_matmul_f32") for k in (8, 64)}
+    finally:
+        arena.free()
+    print(ms)
+    assert ms[8] < 0.8 * ms[64], ms
+
+
