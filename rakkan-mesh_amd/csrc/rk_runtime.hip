@@ -108,6 +108,8 @@ void add_used(rk_device *d, int64_t bytes) {
     d->used += bytes;
 }
 
+static bool overlap(const float *a, int64_t na, const float *b, int64_t nb) { return a < b + nb && b < a + na; }
+
 // Products of n matrices sharing cols with one input: each run of up to
 // three matrices of one format is one launch. Inputs up to 8192 wide that
 // are 16-byte aligned are quantized by every workgroup into LDS (no extra
@@ -188,7 +190,10 @@ int enqueue_matvecs(rk_device *d, int32_t n, rk_matrix *const *ms, float *const 
                          reinterpret_cast<const uint8_t *>(q.qx), q.xs, mx_floats ? x : nullptr, outs[i], ms[i]->raw != 0, s);
     }
     // float32 / bfloat16 matrices take x as it is (internal/gpu/batch.go:
-    // 263-264: no quantized input), up to three of a format a launch
+    // 263-264: no quantized input), up to three of a format a launch. The
+    // launches of a call run one after another, so a matrix whose output
+    // overlaps the input or another's output has a launch of its own: those
+    // after it read what it wrote, and the last output stands.
     for (int kind : {RK_F32, RK_BF16}) {
         DenseMat dm[kDenseMats];
         int k = 0;
@@ -200,8 +205,12 @@ int enqueue_matvecs(rk_device *d, int32_t n, rk_matrix *const *ms, float *const 
         };
         for (int i = 0; i < n; i++) {
             if (ms[i]->kind != kind) continue;
+            const bool over_x = overlap(outs[i], ms[i]->rows, x, cols);
+            bool over = over_x;
+            for (int j = 0; j < k; j++) over = over || overlap(outs[i], ms[i]->rows, dm[j].out, dm[j].rows);
+            if (over) flush();
             dm[k++] = DenseMat{ms[i]->w, outs[i], ms[i]->rows};
-            if (k == kDenseMats) flush();
+            if (over_x || k == kDenseMats) flush();
         }
         flush();
     }

@@ -187,3 +187,39 @@ def test_dense_parts(dev, kind, cols):
         for m in ms:
             m.free()
     assert dev.used == 0
+
+
+@pytest.mark.parametrize("kind", [rkhip.F32, rkhip.BF16])
+def test_dense_outputs_that_overlap(dev, kind):
+    """Matrices of one call run in order: the last output at an offset
+    stands, and a matrix reads what one before it wrote into the input."""
+    rng = np.random.default_rng(9 + kind)
+    cols, rows = 320, [1, 700, 700, 3]
+    x = rng.normal(0, 1, cols).astype(np.float32)
+    ws = [rng.normal(0, 1, r * cols).astype(np.float32) for r in rows]
+    if kind == rkhip.BF16:
+        ws = [to_bf16(w) for w in ws]
+    ms = [dev.upload(kind, r, cols, w) for r, w in zip(rows, ws)]
+    ref = oracle.matvec32 if kind == rkhip.F32 else oracle.matvec_bf16
+    arena = dev.arena(4096, 8192)
+    try:
+        for _ in range(20):
+            b = arena.begin()
+            b.write(0, x)
+            b.matvecs(ms, [1024, 2048, 2048, 3072], 0)  # the second and third at one offset
+            got = [np.asarray(b.read(o, r)) for o, r in ((1024, 1), (2048, 700), (3072, 3))]
+            b.matvecs(ms, [7, 1024, 2048, 3072], 0)     # the first into the input's word 7
+            after = [np.asarray(b.read(o, r)) for o, r in ((7, 1), (1024, 700), (2048, 700), (3072, 3))]
+            b.submit()
+            for g, i in zip(got, (0, 2, 3)):
+                same_bits(g, ref(ws[i], x, rows[i], cols), f"matrix {i}")
+            y = x.copy()
+            y[7] = ref(ws[0], x, 1, cols)[0]
+            same_bits(after[0], y[7:8], "the input's word")
+            for i in (1, 2, 3):
+                same_bits(after[i], ref(ws[i], y, rows[i], cols), f"matrix {i} of the changed input")
+    finally:
+        arena.free()
+        for m in ms:
+            m.free()
+    assert dev.used == 0
