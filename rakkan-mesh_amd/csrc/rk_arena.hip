@@ -360,9 +360,9 @@ int rk_batch_quantize_fp8(rk_batch *b, int64_t in, int64_t n) {
 }
 
 // internal/gpu/dsbatch.go:142-172 ExpertMatVecs: one launch over the slots,
-// which quantizes the inputs itself; inputs off 16 bytes, or in the words
-// from the first output to the last, are quantized into the scratch first
-// (input k at k·cols codes).
+// which quantizes the inputs itself; inputs off 16 bytes, in the words from
+// the first output to the last, or of more weights than that pays for, are
+// quantized into the scratch first (input k at k·cols codes).
 int rk_batch_expert_matvecs(rk_batch *b, rk_matrix *m, int64_t per_expert, int64_t ids, int32_t slots, int64_t in,
                             int64_t in_stride, int32_t div, int64_t out, int64_t out_stride) {
     if (!b) return RK_ERR_ARGS;
@@ -393,7 +393,8 @@ int rk_batch_expert_matvecs(rk_batch *b, rk_matrix *m, int64_t per_expert, int64
     hipStream_t s = d->stream;
     // (every span above lies in the arena, so neither product overflows)
     const int64_t x_last = (inputs - 1) * in_stride, o_last = (slots - 1) * out_stride;
-    const bool floats = mx_takes_floats(x + std::min<int64_t>(x_last, 0), std::abs(x_last) + cols, in_stride,
+    const bool floats = mx_floats_pay(slots * per_expert * cols, inputs, cols, 0, 1) &&
+                        mx_takes_floats(x + std::min<int64_t>(x_last, 0), std::abs(x_last) + cols, in_stride,
                                         o + std::min<int64_t>(o_last, 0), std::abs(o_last) + per_expert);
     if (!floats) {
         ProfScope p(d, s, "act_fp8");

@@ -30,6 +30,10 @@ void mx_fp4_pack_scales(const uint8_t *e8m0, int64_t rows, int64_t cols, uint8_t
 // them stride apart) lie on 16 bytes and share no byte with the out_n floats
 // it writes, which other workgroups may not have read yet.
 bool mx_takes_floats(const float *x, int64_t n, int64_t stride, const float *out, int64_t out_n);
+// Whether that is also faster than a launch that quantizes each input first:
+// `weights` in all, of `inputs` inputs of cols; of one input, over fp8 E4M3
+// and fp4 E2M1 products (expert slots of one matrix: one product).
+bool mx_floats_pay(int64_t weights, int64_t inputs, int64_t cols, int fp8, int fp4);
 
 // internal/num/mx.go:282-334 MatVecFP8 / MatVecFP4 of an input quantized by
 // launch_act_fp8 (codes xc, scales xs): out[r] for rows rows; w E4M3

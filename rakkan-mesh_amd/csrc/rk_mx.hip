@@ -669,6 +669,20 @@ bool mx_takes_floats(const float *x, int64_t n, int64_t stride, const float *out
     return x0 % 16 == 0 && stride % 4 == 0 && (x1 <= o0 || o1 <= x0);
 }
 
+// The launch and its gap are 2 us a call; quantizing inside costs each product
+// a wait (0.5 us E4M3, 1 us E2M1) and then time by its weights, and a row of
+// several chunks waits in each. Measured (us, inside and with the launch):
+// E4M3 6553 x 5120 11.1 and 11.5, 13107 x 5120 17.2 and 16.8, 129280 x 5120 124
+// and 107, 3 x 3276 x 5120 20.8 and 21.0, 1024 x 32768 19.2 and 20.2, 1024 x
+// 65536 36.6 and 35.8; E2M1 13107 x 5120 12.4 and 13.7, 16384 x 8192 19.5 and
+// 19.2, 2 x 16384 x 1024 13.0 and 13.4, 3 x 16384 x 1024 19.2 and 18.6, 512 x
+// 131072 50.2 and 46.4; experts of 2304 x 5120, six slots of one input 12.7
+// and 14.0, 32 of one 44.5 and 43.7, 64 of eight 84.5 and 97.4.
+bool mx_floats_pay(int64_t weights, int64_t inputs, int64_t cols, int fp8, int fp4) {
+    const int64_t most = (int64_t)(inputs > 1 || fp8 == 0 ? 80 : 48) << 20;  // weights an input
+    return cols <= 32768 && weights <= most * inputs && fp8 + fp4 <= (fp4 > 0 ? 2 : 3);
+}
+
 void launch_mx_matvec(bool fp4, const uint8_t *w, const uint8_t *ws, int64_t rows, int64_t cols, const uint8_t *xc,
                       const float *xs, const float *x, float *out, bool raw, hipStream_t s) {
     const MxShape sh = mx_shape(fp4, (int)(cols / 32));

@@ -167,17 +167,19 @@ int enqueue_matvecs(rk_device *d, int32_t n, rk_matrix *const *ms, float *const 
     // E4M3 / E2M1 matrices, one launch each, the input quantized to E4M3 with
     // block scales (internal/gpu/batch.go:221-233 QuantizeFP8) inside it: a
     // lane quantizes only its own slice, by the hardware's conversion, while
-    // the weights are on their way. An input off 16 bytes, or one that a
-    // matrix's output overlaps, is quantized once into the scratch first; so
-    // is one of more than three matrices (a product takes up to 2.3 us longer
-    // for it, the launch and its gap about 7).
+    // the weights are on their way. An input off 16 bytes, one that a matrix's
+    // output overlaps, and one of products for which the launch is faster
+    // (mx_floats_pay) is quantized once into the scratch first.
     bool mx_floats = true, mx_quantized = false;
-    int mx_count = 0;
+    int fp8 = 0, fp4 = 0;
+    int64_t mx_weights = 0;
     for (int i = 0; i < n; i++) {
         mx_floats = mx_floats && mx_takes_floats(x, cols, 0, outs[i], ms[i]->rows);
-        mx_count += ms[i]->kind == RK_FP8 || ms[i]->kind == RK_FP4;
+        fp8 += ms[i]->kind == RK_FP8;
+        fp4 += ms[i]->kind == RK_FP4;
+        if (ms[i]->kind == RK_FP8 || ms[i]->kind == RK_FP4) mx_weights += ms[i]->rows * cols;
     }
-    mx_floats = mx_floats && mx_count <= 3;
+    mx_floats = mx_floats && mx_floats_pay(mx_weights, 1, cols, fp8, fp4);
     for (int i = 0; i < n; i++) {
         if (ms[i]->kind != RK_FP8 && ms[i]->kind != RK_FP4) continue;
         if (!mx_floats && !mx_quantized) {

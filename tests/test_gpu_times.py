@@ -45,3 +45,21 @@ def test_tensor_positions_past_k_cost_nothing(dev, transposed):
     assert ms[8] < 0.8 * ms[64], ms
 
 
+@pytest.mark.parametrize("kind,rows,cols,n,inside", [
+    (rkhip.FP8, 4096, 1024, 3, True), (rkhip.FP8, 64, 65536, 1, False), (rkhip.FP8, 16384, 4096, 1, False),
+    (rkhip.FP4, 4096, 1024, 2, True), (rkhip.FP4, 64, 1024, 3, False), (rkhip.FP4, 64, 65536, 1, False),
+    (rkhip.FP4, 32768, 4096, 1, False)])
+def test_block_scaled_products_quantize_where_it_pays(dev, kind, rows, cols, n, inside):
+    """The input's quantize launch, by the weights that would quantize it
+    again: inside the products for the smaller calls only."""
+    w = np.zeros(rows * cols // (1 if kind == rkhip.FP8 else 2), np.uint8)
+    s = np.full((rows + 31) // 32 * (cols // 32) if kind == rkhip.FP8 else rows * cols // 32, 120, np.uint8)
+    ms = [dev.upload_mx(kind, rows, cols, w, s) for _ in range(n)]
+    try:
+        prof = profile(dev, lambda: dev.matvecs(ms, np.ones(cols, np.float32)))
+    finally:
+        for m in ms:
+            m.free()
+    assert ("act_fp8" in prof) == (not inside), prof
+
+
