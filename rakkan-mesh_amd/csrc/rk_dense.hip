@@ -33,6 +33,7 @@
 // sums a lane, four rows a wave (15.5) and 1, 2 and 8 waves a workgroup.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "rk_dense.h"
 #include "rk_dev.h"
@@ -46,9 +47,7 @@ constexpr int kDensePart = 512;  // elements of a row (16 steps) in a ring part
 constexpr int kDenseX = 8192;    // input elements staged at a time
 constexpr int kDenseRing = 2;    // parts of a wave's ring
 
-typedef int rk_v2i __attribute__((ext_vector_type(2)));
 typedef float rk_v2f __attribute__((ext_vector_type(2)));
-typedef float rk_v4f __attribute__((ext_vector_type(4)));
 
 struct DenseArgs {
     DenseMat m[kDenseMats];
@@ -56,6 +55,7 @@ struct DenseArgs {
     const float *x;
     int64_t row_elems;
     int32_t cols, waves;        // waves a workgroup
+    int32_t groups;             // dense_narrow_kernel: groups of four rows a wave
 };
 
 __device__ __forceinline__ uint32_t lds_off(void *p) { return (uint32_t)(uintptr_t)lds_ptr(p); }
@@ -65,19 +65,14 @@ __device__ __forceinline__ void load_lds16(const uint8_t *from, uint8_t *to) {
     __builtin_amdgcn_global_load_lds(from, lds_ptr(to), 16, 0, kAuxStream);
 }
 
-// Waits until at most n·NI of the wave's loads are in flight (n <= 7).
+// Waits for the wave's loads, except (more) the NI of the ring's other part.
 template <int NI>
-__device__ __forceinline__ void wait_parts(int n) {
-    switch (n) {  // uniform
-    case 0: __builtin_amdgcn_s_waitcnt(vmcnt_wait(0)); break;
-    case 1: __builtin_amdgcn_s_waitcnt(vmcnt_wait(NI)); break;
-    case 2: __builtin_amdgcn_s_waitcnt(vmcnt_wait(2 * NI)); break;
-    case 3: __builtin_amdgcn_s_waitcnt(vmcnt_wait(3 * NI)); break;
-    case 4: __builtin_amdgcn_s_waitcnt(vmcnt_wait(4 * NI)); break;
-    case 5: __builtin_amdgcn_s_waitcnt(vmcnt_wait(5 * NI)); break;
-    case 6: __builtin_amdgcn_s_waitcnt(vmcnt_wait(6 * NI)); break;
-    default: __builtin_amdgcn_s_waitcnt(vmcnt_wait(7 * NI)); break;
-    }
+__device__ __forceinline__ void wait_part(bool more) {
+    static_assert(kDenseRing == 2, "one part in flight past the one waited for");
+    if (more)  // uniform
+        __builtin_amdgcn_s_waitcnt(vmcnt_wait(NI));
+    else
+        __builtin_amdgcn_s_waitcnt(vmcnt_wait(0));
     asm volatile("" ::: "memory");
 }
 
@@ -210,7 +205,7 @@ __global__ __launch_bounds__(256) void dense_matvec_kernel(DenseArgs a) {
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
         }
-        wait_parts<D::NI>(min(S - 1, parts - 1 - c));
+        wait_part<D::NI>(c + 1 < parts);
         DensePart<BF> t;
         t.read(wo + (c % S) * D::PART, xo + 4 * c0);
         if (c + S < parts) fetch(c + S);  // into the part just read
@@ -234,8 +229,118 @@ __global__ __launch_bounds__(256) void dense_matvec_kernel(DenseArgs a) {
     if (l == 0 && r0 + g < rows) a.m[mi].out[r0 + g] = res;
 }
 
+// v of the lane N up in its row of 16 (the last N lanes: another's).
+template <int N>
+__device__ __forceinline__ float row_up(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x100 + N, 0xf, 0xf, true));
+}
+
+// Rows of at most ST steps (narrow ones): lane l of the 16 of a row keeps the
+// running sums 2l and 2l + 1, four rows a wave, and holds the row and its own
+// input elements in registers; a wave takes a.groups groups of four rows, the
+// next one's loads in flight during the sums. The ring above reads whole parts
+// of 512 elements and a wave ends after two rows: bounded by latency and by
+// the number of waves. Measured (us, ring and this): bfloat16 32000 x 288 9.8
+// and 5.3, 16000 x 384 6.3 and 4.5, 1000000 x 32 201 and 23, float32 32000 x
+// 288 12.7 and 7.1, 128000 x 32 34.7 and 8.0.
+template <bool BF, int ST>
+__global__ __launch_bounds__(256) void dense_narrow_kernel(DenseArgs a) {
+    typedef typename std::conditional<BF, uint32_t, float2>::type W;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int l = lane & 15, g = lane >> 4;
+    const int steps = (int)a.row_elems >> 5;
+    const int64_t gw = (int64_t)blockIdx.x * a.waves + wv;
+    const int mi = (gw >= a.first[1] ? 1 : 0) + (gw >= a.first[2] ? 1 : 0);
+    const int64_t rows = a.m[mi].rows, r0 = (gw - a.first[mi]) * (4 * a.groups);
+    if (r0 >= rows) return;
+    const int64_t rw = a.row_elems * (BF ? 2 : 4) / (int64_t)sizeof(W);  // a row's loads
+    const W *w = static_cast<const W *>(a.m[mi].w) + l;
+    const int ng = (int)min((int64_t)a.groups, (rows - r0 + 3) >> 2);
+    W wc[ST];
+    auto load = [&](int64_t r) {
+        const W *p = w + min(r + g, rows - 1) * rw;
+#pragma unroll
+        for (int m = 0; m < ST; m++) wc[m] = p[16 * min(m, steps - 1)];
+    };
+    load(r0);
+    // the lane's input elements, zeros past cols (odd widths in the last step
+    // alone: a lane there reads the last pair of the input)
+    float2 x[ST];
+    if (a.cols == a.row_elems) {  // uniform
+#pragma unroll
+        for (int m = 0; m < ST; m++) __builtin_memcpy(&x[m], a.x + 32 * min(m, steps - 1) + 2 * l, 8);
+    } else {
+        const int i = 32 * (steps - 1) + 2 * l, o = min(i, a.cols - 2);
+        float2 v = {0.0f, a.x[0]};
+        if (a.cols > 1) __builtin_memcpy(&v, a.x + o, 8);
+        if (steps > 1)
+#pragma unroll
+            for (int m = 0; m < ST - 1; m++) __builtin_memcpy(&x[m], a.x + 32 * min(m, steps - 2) + 2 * l, 8);
+        const float2 t = {i == o ? v.x : i == o + 1 ? v.y : 0.0f, i == o ? v.y : 0.0f};
+#pragma unroll
+        for (int m = 0; m < ST; m++)
+            if (m == steps - 1) x[m] = t;
+    }
+    for (int i = 0; i < ng; i++) {
+        W wt[ST];
+#pragma unroll
+        for (int m = 0; m < ST; m++) wt[m] = wc[m];
+        const int64_t r = r0 + 4 * i;
+        if (i + 1 < ng) load(r + 4);
+        float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+        for (int m = 0; m < ST; m++)
+            if (m < steps) {  // uniform
+                if constexpr (BF) {
+                    s0 += __uint_as_float(wt[m] << 16) * x[m].x;
+                    s1 += __uint_as_float(wt[m] & 0xffff0000u) * x[m].y;
+                } else {
+                    s0 += wt[m].x * x[m].x;
+                    s1 += wt[m].y * x[m].y;
+                }
+            }
+        const float v0 = s0 + row_up<4>(s0), v1 = s1 + row_up<4>(s1);
+        const float e0 = v0 + row_up<8>(v0), e1 = v1 + row_up<8>(v1);
+        const float p = e0 + e1;
+        const float q = p + row_up<1>(p);
+        const float res = q + row_up<2>(q);
+        if (l == 0 && r + g < rows) a.m[mi].out[r + g] = res;
+    }
+}
+
+template <bool BF, int ST>
+void launch_narrow_t(DenseArgs a, int n, hipStream_t s) {
+    int64_t groups = 0, waves = 0;
+    for (int i = 0; i < n; i++) groups += (a.m[i].rows + 3) / 4;
+    // up to four groups a wave while 2048 waves are left (32000 x 288: one 7.4
+    // us, two 5.8, four 5.3), more once 8192 are (1000000 x 32: 8192 waves 23,
+    // 2048 waves 54)
+    a.groups = (int)std::max<int64_t>((groups + 8191) / 8192, std::min<int64_t>(4, (groups + 2047) / 2048));
+    for (int i = 0; i < kDenseMats; i++) {
+        a.first[i] = i < n ? waves : INT64_MAX;
+        if (i < n) waves += (a.m[i].rows + 4 * a.groups - 1) / (4 * a.groups);
+    }
+    a.waves = (int)std::min<int64_t>(4, std::max<int64_t>(1, waves / 256));
+    RK_LAUNCH((dense_narrow_kernel<BF, ST>), dim3((unsigned)((waves + a.waves - 1) / a.waves)),
+              dim3((unsigned)(64 * a.waves)), 0, s, a);
+}
+
 template <bool BF>
 void launch_dense_t(DenseArgs a, int n, hipStream_t s) {
+    // Wider float32 rows hold too many registers for it (4000 x 512 4.3 us, by
+    // the ring 3.7; 24000 x 512 10.3 and 10.0).
+    constexpr int widest = BF ? 16 : 14;  // steps
+    if (a.row_elems <= 32 * widest) {
+        if (a.row_elems <= 128)
+            launch_narrow_t<BF, 4>(a, n, s);
+        else if (a.row_elems <= 288)
+            launch_narrow_t<BF, 9>(a, n, s);
+        else if (a.row_elems <= 384)
+            launch_narrow_t<BF, 12>(a, n, s);
+        else
+            launch_narrow_t<BF, widest>(a, n, s);
+        return;
+    }
     typedef DenseShape<BF> D;
     static std::once_flag once;
     std::call_once(once, [] {

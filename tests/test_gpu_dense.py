@@ -223,3 +223,38 @@ def test_dense_outputs_that_overlap(dev, kind):
         for m in ms:
             m.free()
     assert dev.used == 0
+
+
+# Narrow rows (16 lanes a row, in registers): widths about each instance's
+# steps, odd ones (float32), and enough rows for waves of several groups of
+# four, the last of them partial.
+@pytest.mark.parametrize("cols", [1, 3, 31, 33, 34, 128, 130, 258, 288, 290, 383, 384, 386, 416, 418, 448, 450, 480])
+@pytest.mark.parametrize("kind", [rkhip.F32, rkhip.BF16])
+def test_dense_narrow_rows(dev, kind, cols):
+    cols += cols % 2 if kind == rkhip.BF16 else 0
+    rng = np.random.default_rng(cols + kind)
+    rows = [40003, 6, 9001] if cols in (34, 130, 290, 416) else [1030, 1, 7]
+    x = awkward(rng, cols)
+    x[rng.integers(0, cols)] = np.inf
+    ws = [awkward(rng, r * cols, 0.1) for r in rows]
+    if kind == rkhip.BF16:
+        ws = [to_bf16(w) for w in ws]
+    ms = [dev.upload(kind, r, cols, w) for r, w in zip(rows, ws)]
+    ref = oracle.matvec32 if kind == rkhip.F32 else oracle.matvec_bf16
+    want = [ref(w, x, r, cols) for r, w in zip(rows, ws)]
+    offs = np.cumsum([cols + 4] + rows).tolist()
+    arena = dev.arena(offs[-1], 2 * offs[-1])
+    try:
+        for at in (0, 1, 4):
+            b = arena.begin()
+            b.write(at, x)
+            b.matvecs(ms, offs[:3], at)
+            got = [b.read(o, r) for o, r in zip(offs, rows)]
+            b.submit()
+            for y, w in zip(got, want):
+                same_bits(np.asarray(y), w, f"{cols} columns, input at word {at}")
+    finally:
+        arena.free()
+        for m in ms:
+            m.free()
+    assert dev.used == 0

@@ -63,3 +63,21 @@ def test_block_scaled_products_quantize_where_it_pays(dev, kind, rows, cols, n, 
     assert ("act_fp8" in prof) == (not inside), prof
 
 
+@pytest.mark.parametrize("kind", [rkhip.BF16, rkhip.F32])
+def test_narrow_dense_rows(dev, kind):
+    """128000 rows of 32 values against as many of 512."""
+    ms = {}
+    for cols in (32, 512):
+        m = dev.upload(kind, 128000, cols, np.zeros(128000 * cols, np.uint16 if kind == rkhip.BF16 else np.float32))
+        arena = dev.arena(cols + 128000, 64)
+        try:
+            name = "matvec_bf16" if kind == rkhip.BF16 else "matvec_f32"
+            ms[cols] = least_ms(dev, lambda: dev.matvecs_device([m], [arena.device_ptr(cols)], arena.device_ptr(0), cols),
+                                name)
+        finally:
+            arena.free()
+            m.free()
+    print(ms)
+    assert ms[32] < 0.75 * ms[512], ms
+
+
