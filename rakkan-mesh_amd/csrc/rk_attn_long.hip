@@ -227,7 +227,7 @@ bool launch_att_scores_long(const float *q, const float *keys, float *att, int32
         bt.q_stride % 4 != 0 || ((reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(q)) & 15) != 0 ||
         bt.cache_stride % 4 != 0)
         return false;
-    const int npos = ctl || bt.pos ? ctx : bt.pos0 + bt.tokens;
+    const int npos = att_positions(ctl, bt, ctx);
     const dim3 grid(kv_heads, (npos + kLongTile - 1) / kLongTile, ctl ? 1 : bt.tokens);
     RK_LAUNCH(att_scores_long_kernel, grid, dim3(256), 0, s, q, keys, att, att_stride, ctl, bt, kv_mul, kv_dim, inv_sqrt);
     return true;

@@ -150,6 +150,13 @@ __device__ __forceinline__ int att_position(const int32_t *ctl, const AttBatch &
     return ctl ? ctl[kCtlPos] : (bt.pos ? bt.pos[z] : bt.pos0 + z);
 }
 
+// Positions an attention launch covers (ctx: the caches' length): those of a
+// prompt's tokens, or, a decode step or independent sequences (positions read
+// on the device), all of them.
+inline int att_positions(const int32_t *ctl, const AttBatch &bt, int ctx) {
+    return ctl ? ctx : bt.groups ? bt.max_pos : bt.pos ? ctx : bt.pos0 + bt.tokens;
+}
+
 // Attention of one position over a stage's cache (internal/llm/model.go:
 // 575-591), position and length read from ctl (or, ctl null, a batch):
 // scores, then softmax and the weighted values (f32 out).

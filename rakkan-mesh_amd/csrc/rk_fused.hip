@@ -637,9 +637,10 @@ void launch_att_scores(const float *q, const float *keys, float *att, int32_t at
         return;
     }
     if (launch_att_scores_long(q, keys, att, att_stride, ctl, bt, ctx, heads, kv_heads, hs, kv_dim, inv_sqrt, s)) return;
-    // decode and independent sequences: positions up to ctx (tiles past a
-    // token's position exit); a batch: up to its last token's
-    const int npos = ctl || bt.pos ? ctx : bt.pos0 + bt.tokens;
+    // tiles past a token's position exit: 256 prompt tokens of 32 heads of 64
+    // in a context of 8192 launch a million of them a layer if the context
+    // gives the count (111 us against 7.7 for eight prompts of 17)
+    const int npos = att_positions(ctl, bt, ctx);
     const dim3 grid(heads, (npos + kScoreTile - 1) / kScoreTile, ctl ? 1 : bt.tokens);
     if (hs == 128)
         RK_LAUNCH(att_scores_kernel<128>, grid, dim3(256), 0, s, q, keys, att, att_stride, ctl, bt, heads / kv_heads,

@@ -81,3 +81,28 @@ def test_narrow_dense_rows(dev, kind):
     assert ms[32] < 0.75 * ms[512], ms
 
 
+def test_shared_prompts_scores_do_not_grow_with_the_context(dev):
+    """Heads of 64: a scores workgroup for each position up to the furthest
+    prompt's, not up to the context."""
+    c = Config(dim=64, hidden=64, layers=1, heads=32, kv_heads=2, head_dim=64, vocab=50, seq_len=8192, dtype="q8_0")
+    m = coded_model(c, 5, 1e-3, 1e-2)
+    prompts = [[int(t) for t in np.random.default_rng(z).integers(0, c.vocab, 17)] for z in range(8)]
+    ms = {}
+    for ctx in (256, 8192):
+        layers, mats = upload_layers(dev, m)
+        emb = dev.upload(m.embed.kind, m.embed.rows, m.embed.cols, m.embed.q, m.embed.scales)
+        cos, sin = m.rope(ctx)
+        st = rkhip.Stage(dev, c.dim, c.hidden, c.heads, c.kv_heads, ctx, layers, cos, sin, head_dim=c.head_dim,
+                         norm_eps=float(c.eps()), seqs=len(prompts))
+        try:
+            st.set_head(emb, emb, m.rms_final)
+            st.seqs_start(prompts)
+            ms[ctx] = least_ms(dev, lambda: st.seqs_start(prompts), "att_scores")
+        finally:
+            st.free()
+            emb.free()
+            for mt in mats:
+                mt.free()
+    assert ms[8192] < 2 * ms[256], ms
+
+
