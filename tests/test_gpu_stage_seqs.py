@@ -90,3 +90,18 @@ def test_prompts_share_batches(dev, qk_norm, dtype):
             same_bits(lg[k, z], want_l[k], f"sequence {z} (prompt {len(p)}), step {k}")
         assert toks[z] == want_t, f"sequence {z} tokens"
     assert dev.used == 0
+
+
+def test_most_sequences(dev):
+    """256 sequences of up to four tokens: a group each, empty prompts among
+    them, over two batches."""
+    c = Config(dim=64, hidden=64, layers=1, heads=2, kv_heads=1, vocab=50, seq_len=8, head_dim=32, dtype="q8_0")
+    m = coded_model(c, seed=8, scale_lo=1e-3, scale_hi=1e-2)
+    rng = np.random.default_rng(6)
+    prompts = [[int(t) for t in rng.integers(0, c.vocab, n)] for n in rng.integers(1, 5, 256)]
+    lg, toks = seqs_generate(dev, m, prompts, 1, 8)
+    for z, p in enumerate(prompts):
+        want_t, want_l = oracle_generate(m, p, 1, 8)
+        same_bits(lg[0, z], want_l[0], f"sequence {z} (prompt {len(p)})")
+        assert toks[z] == want_t, f"sequence {z} tokens"
+    assert dev.used == 0
