@@ -15,8 +15,10 @@
 // odd one, a scan, again after each thread that leaves the binade) measured
 // slower: 2.7 us a scan, and rows whose terms grow towards the last position
 // leave a binade every few threads (35-56 us against the chain's 22).
+#include <algorithm>
 #include <mutex>
 
+#include "rk_attn_reg.h"
 #include "rk_dev.h"
 #include "rk_fused.h"
 
@@ -27,6 +29,8 @@ namespace {
 constexpr int kLongHs = 128;       // head size of the scores kernel
 constexpr int kLongTile = 64;      // positions a scores workgroup
 constexpr int kLongMaxMul = 16;    // query heads a kv head
+constexpr int kLongSplit = 4;      // scores workgroups a kv head and tile, at most
+constexpr int kLongWgs = 512;      // scores workgroups that keep the chip busy
 constexpr int kLongThreads = 512;  // values: waves 0-3 (0 adds), waves 4-7 load and multiply
 constexpr int kLongWaves = kLongThreads / 64;
 constexpr int kLongSlice = 32;     // elements a workgroup
@@ -34,19 +38,28 @@ constexpr int kLongChunk = 256;    // positions a product tile
 
 }  // namespace
 
-// Scores of kLongTile positions for the query heads of one kv head (size
-// 128): thread (position tid/4, part tid%4) keeps its key's elements 8·part
-// .. +7 of each 32-element step in registers and runs the heads over them,
-// as quad_dot32 (the running sums j = 8·part .. +7, combined by DPP).
+// Scores of kLongTile positions for query heads of one kv head (size 128):
+// thread (position tid/4, part tid%4) keeps its key's elements 8·part .. +7 of
+// each 32-element step in registers and runs the heads over them, as
+// quad_dot32 (the running sums j = 8·part .. +7, combined by DPP). A kv head's
+// `split` workgroups share its query heads while the positions so far leave
+// workgroups of the chip idle; from there on the first takes them all.
 __global__ __launch_bounds__(256) void att_scores_long_kernel(const float *q, const float *keys, float *att,
                                                               int32_t att_stride, const int32_t *ctl, AttBatch bt,
-                                                              int kv_mul, int kv_dim, float inv_sqrt) {
+                                                              int kv_heads, int kv_mul, int split, int kv_dim,
+                                                              float inv_sqrt) {
     __shared__ __align__(16) float sq[kLongMaxMul * kLongHs];
     const int z = blockIdx.z;
     const int T = att_position(ctl, bt, z) + 1;
     const int t0 = blockIdx.y * kLongTile;
     if (t0 >= T) return;
-    const int g = blockIdx.x, h0 = g * kv_mul;
+    const int g = (int)blockIdx.x / split, part_of = (int)blockIdx.x % split;
+    const int whole = kv_heads * ((T + kLongTile - 1) / kLongTile) * (int)gridDim.z;  // one a kv head and tile
+    const int parts = min(split, max(1, kLongWgs / whole));
+    const int share = (kv_mul + parts - 1) / parts;
+    const int m0 = part_of * share, m1 = min(kv_mul, m0 + share);  // its heads
+    if (m0 >= kv_mul) return;
+    const int h0 = g * kv_mul;
     const int part = threadIdx.x & 3, t = t0 + (threadIdx.x >> 2);
     const float *kt = keys + att_cache(bt, z) + (int64_t)min(t, T - 1) * kv_dim + (int64_t)g * kLongHs + 8 * part;
     float4 k0[kLongHs / 32], k1[kLongHs / 32];
@@ -56,11 +69,11 @@ __global__ __launch_bounds__(256) void att_scores_long_kernel(const float *q, co
         k1[st] = *reinterpret_cast<const float4 *>(kt + 32 * st + 4);
     }
     const float *qh = q + (int64_t)z * bt.q_stride + (int64_t)h0 * kLongHs;
-    for (int i = threadIdx.x; i < kv_mul * (kLongHs / 4); i += 256)
+    for (int i = m0 * (kLongHs / 4) + threadIdx.x; i < m1 * (kLongHs / 4); i += 256)
         reinterpret_cast<float4 *>(sq)[i] = reinterpret_cast<const float4 *>(qh)[i];
     __syncthreads();
     att += (int64_t)z * bt.att_stride;
-    for (int m = 0; m < kv_mul; m++) {
+    for (int m = m0; m < m1; m++) {
         float s[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) s[k] = 0.0f;
@@ -92,7 +105,9 @@ __global__ __launch_bounds__(256) void att_scores_long_kernel(const float *q, co
 // x of token y): Go max, e_t = Exp32(s_t - max), the sum, inv = Recip32(sum),
 // then out_i = Σ_t (e_t·inv)·v_t,i in t order from +0. Chunk c's products
 // stand transposed and swizzled in tile c mod 2 while wave 0 adds them; waves
-// 4-7 meanwhile write chunk c+1's from registers and request chunk c+3.
+// 4-7 meanwhile write chunk c+1's from registers and request chunk c+3. A
+// position that sees at most kVrMaxCtx takes att_values_reg_body (position 50
+// of a context of 8192: 7.0 us here, 4.9 there).
 __global__ __launch_bounds__(kLongThreads) void att_values_long_kernel(const float *att, int32_t att_stride,
                                                                        const float *vals, float *out,
                                                                        const int32_t *ctl, AttBatch bt, int kv_mul,
@@ -106,6 +121,11 @@ __global__ __launch_bounds__(kLongThreads) void att_values_long_kernel(const flo
     float *tiles = smem + ctx_pad;  // [2][32][kLongChunk] products, swizzled rows
     const int z = blockIdx.y;
     const int T = att_position(ctl, bt, z) + 1;
+    if (T <= kVrMaxCtx) {  // uniform
+        att_values_reg_body<false>(att, att_stride, vals, out, ctl, bt, kv_mul, hs, kv_dim, nsl, ctx_pad, qx, xs, xsum,
+                                   blockIdx.x, z, nullptr, 0);
+        return;
+    }
     const int nch = (T + kLongChunk - 1) / kLongChunk;
     const int h = blockIdx.x / nsl, e0 = (blockIdx.x % nsl) * kLongSlice;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -121,25 +141,32 @@ __global__ __launch_bounds__(kLongThreads) void att_values_long_kernel(const flo
                 v[q][j] = *reinterpret_cast<const float4 *>(
                     vb + (int64_t)min(c * kLongChunk + 4 * (pq + 32 * q) + j, T - 1) * kv_dim);
     };
+    // the head's scores, eight in flight a thread; the first before the values
+    // (loads arrive in order)
+    const float *ah = att + (int64_t)z * bt.att_stride + (int64_t)h * att_stride;
+    float sv[8];
+    auto scores = [&](int t0) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) sv[k] = ah[min(t0 + tid + k * kLongThreads, T - 1)];
+    };
+    scores(0);
     if (wave >= 4) {
         load(va, 0);
         load(vc, 1);
     }
-    // the head's scores, eight in flight a thread
-    const float *ah = att + (int64_t)z * bt.att_stride + (int64_t)h * att_stride;
-    float m = ah[0];
-    for (int t0 = 0; t0 < T; t0 += 8 * kLongThreads) {
-        float v[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) v[k] = ah[min(t0 + tid + k * kLongThreads, T - 1)];
+    float m = sv[0];
+    for (int t0 = 0;;) {
 #pragma unroll
         for (int k = 0; k < 8; k++) {
             const int t = t0 + tid + k * kLongThreads;
             if (t < T) {
-                sa[t] = v[k];
-                m = gomax(m, v[k]);
+                sa[t] = sv[k];
+                m = gomax(m, sv[k]);
             }
         }
+        t0 += 8 * kLongThreads;
+        if (t0 >= T) break;
+        scores(t0);
     }
     m = wave_gomax(m);
     if (lane == 0) s_red[wave] = m;
@@ -177,26 +204,51 @@ __global__ __launch_bounds__(kLongThreads) void att_values_long_kernel(const flo
             acc = swz_chain_sum(tiles + (c & 1) * (kLongSlice * kLongChunk) + lane * kLongChunk,
                                 min(kLongChunk, T - c * kLongChunk), vr_swz(lane), acc);
     };
+    // While five chunks are left each half loads unconditionally (a test
+    // around a load makes the compiler wait there); the last ones load nothing
+    // that nobody reads, for a launch ends when its loads have. (nch >= 5.)
+    int c = 0;
     if (wave >= 4) {
         products(va, 0);
         load(va, 2);
     }
     __syncthreads();
-    for (int c = 0; c < nch; c += 2) {
+    for (; c + 4 < nch; c += 2) {
         if (wave == 0) {
             sums(c);
-        } else if (wave >= 4) {  // (a chunk past the last: products that nothing reads)
+        } else if (wave >= 4) {
             products(vc, c + 1);
             load(vc, c + 3);
         }
         __syncthreads();
         if (wave == 0) {
-            if (c + 1 < nch) sums(c + 1);
+            sums(c + 1);
         } else if (wave >= 4) {
             products(va, c + 2);
             load(va, c + 4);
         }
         __syncthreads();
+    }
+    const bool four = nch - c > 3;  // three or four chunks: vc holds the second, va the third
+    if (wave == 0) {
+        sums(c);
+    } else if (wave >= 4) {
+        products(vc, c + 1);
+        if (four) load(vc, c + 3);
+    }
+    __syncthreads();
+    if (wave == 0)
+        sums(c + 1);
+    else if (wave >= 4)
+        products(va, c + 2);
+    __syncthreads();
+    if (wave == 0)
+        sums(c + 2);
+    else if (wave >= 4 && four)
+        products(vc, c + 3);
+    if (four) {  // uniform
+        __syncthreads();
+        if (wave == 0) sums(c + 3);
     }
     if (wave != 0) return;
     const int64_t base = (int64_t)z * bt.out_stride + (int64_t)h * hs + e0;
@@ -228,8 +280,13 @@ bool launch_att_scores_long(const float *q, const float *keys, float *att, int32
         bt.cache_stride % 4 != 0)
         return false;
     const int npos = att_positions(ctl, bt, ctx);
-    const dim3 grid(kv_heads, (npos + kLongTile - 1) / kLongTile, ctl ? 1 : bt.tokens);
-    RK_LAUNCH(att_scores_long_kernel, grid, dim3(256), 0, s, q, keys, att, att_stride, ctl, bt, kv_mul, kv_dim, inv_sqrt);
+    const int tokens = ctl ? 1 : bt.tokens, tiles = (npos + kLongTile - 1) / kLongTile;
+    // (where the device holds the positions, there may be one tile a token)
+    const int whole = kv_heads * tokens * (ctl || bt.pos ? 1 : tiles);
+    const int split = std::min(std::min(kv_mul, kLongSplit), std::max(1, kLongWgs / whole));
+    const dim3 grid(kv_heads * split, tiles, tokens);
+    RK_LAUNCH(att_scores_long_kernel, grid, dim3(256), 0, s, q, keys, att, att_stride, ctl, bt, kv_heads, kv_mul, split,
+              kv_dim, inv_sqrt);
     return true;
 }
 

@@ -106,3 +106,24 @@ def test_shared_prompts_scores_do_not_grow_with_the_context(dev):
     assert ms[8192] < 2 * ms[256], ms
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd", [(16, 1, 128), (32, 8, 128), (32, 8, 64)])
+def test_early_positions_of_a_long_context(dev, heads, kv_heads, hd):
+    """A decode step at position 40: its attention's scores and values in a
+    context of 4096 positions against one of 1024."""
+    c = Config(dim=64, hidden=64, layers=1, heads=heads, kv_heads=kv_heads, head_dim=hd, vocab=50, seq_len=4096,
+               dtype="q8_0")
+    m = coded_model(c, 5, 1e-3, 1e-2)
+    xs = np.random.default_rng(1).normal(0, 1, (41, c.dim)).astype(np.float32)
+    ms = {}
+    for ctx in (1024, 4096):
+        st, mats = make_stage(dev, m, ctx)
+        try:
+            st.forward(xs[:40], 0)
+            p = [profile(dev, lambda: st.forward(xs[40:], 40)) for _ in range(25)]
+            ms[ctx] = {k: min(x[k][1] for x in p) for k in p[0] if k.startswith("att_")}
+        finally:
+            st.free()
+            for mt in mats:
+                mt.free()
+
+    assert ms[4096]["att_scores"] < 1.35 * ms[1024]["att_scores"], ms
