@@ -1185,7 +1185,15 @@ void launch_att_values(const float *att, int32_t att_stride, const float *vals, 
                   (ctx + 3) & ~3, qx, xs, xsum);
         return;
     }
-    if (launch_att_values_long(att, att_stride, vals, out, ctl, bt, ctx, heads, kv_heads, hs, kv_dim, qx, xs, xsum, s))
+    // Past kVrMaxCtx positions a workgroup of rk_attn_long.hip has a CU to
+    // itself; more of them than CUs are faster by att_values_kernel where its
+    // LDS leaves a CU room for two (up to 3.8 k positions; a prompt's tokens
+    // 1024-1535 of 32 heads of 128, two layers: 8.4 ms against 10.6; a context
+    // of 8192 11.8 and 10.6).
+    const bool two = (int64_t)grid.x * grid.y * grid.z > (cu > 0 ? cu : 256) &&
+                     att_values_lds(ctx, kValChunk) + 1024 <= kMaxLdsBytes / 2;
+    if (!two &&
+        launch_att_values_long(att, att_stride, vals, out, ctl, bt, ctx, heads, kv_heads, hs, kv_dim, qx, xs, xsum, s))
         return;
     if (vec)
         RK_LAUNCH((att_values_kernel<true, kValChunk>), grid, dim3(kValThreads), att_values_lds(ctx, kValChunk), s, att,
