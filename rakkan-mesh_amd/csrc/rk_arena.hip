@@ -39,16 +39,27 @@ struct rk_batch {
     };
     std::vector<PendingRead> reads;
     int err = RK_OK;
+    struct Move {  // n words to dst
+        float *dst;
+        const float *src;
+        int64_t n;
+        hipMemcpyKind kind;
+        const char *what;
+    };
+    Move first{};     // the first operation, a move, while it is the only one
+    int64_t ops = 0;  // operations so far
 };
 
 namespace rk {
 
-// Words that a kernel moves between the arena and the host's staging; longer
-// moves take the copy engine. A batch of one write and one copy, and of one
-// copy and one read, by the engine and by a kernel: 5120 words 22.8 and 23.2
-// us against 18.8 and 18.9, 30720 words 25.5 and 27.2 against 20.9 and 22.4,
-// 262144 words 65.9 and 72.0 against 61.0 and 67.0; from 1048576 words the
-// link decides (write 164 against 167 us).
+// Words of a move between the arena and the host's staging that a kernel
+// makes: up to kBlitWords the runtime's own copy is a kernel too (4096 words
+// four times a batch 27.9 us, by launch_copy 29.0), past kMoveWords the link
+// decides. Between them the runtime takes the copy engine, and a batch of one
+// write and one copy, and of one copy and one read, took 22.8 and 23.2 us
+// against 18.8 and 18.9 at 5120 words, 65.9 and 72.0 against 61.0 and 67.0 at
+// 262144 (1048576: write 164 against 167).
+constexpr int64_t kBlitWords = 4096;
 constexpr int64_t kMoveWords = 1 << 18;
 
 static int latch(rk_batch *b, int code) {
@@ -86,15 +97,36 @@ static int launched(rk_batch *b, const char *what) {
 // the kernels before it, and the kernels after it for the copy, by signals
 // between queues; a kernel that reads or writes the pinned words needs none
 // (a DeepSeek-V4.1-shaped layer's products, two writes and a read: 125.5 ->
-// 94.1 us).
-static int move_words(rk_batch *b, float *dst, const float *src, int64_t n, hipMemcpyKind kind, const char *what) {
-    rk_device *d = b->a->d;
-    if (n <= kMoveWords) {
-        launch_copy(src, dst, n, d->stream);
-        return launched(b, what);
-    }
-    hipError_t e = hipMemcpyAsync(dst, src, (size_t)n * 4, kind, d->stream);
-    return e == hipSuccess ? RK_OK : latch(b, hip_fail(d, e, what));
+// 94.1 us). A batch of a single move has nothing to wait for and is faster by
+// the engine (a write of 5000 words 11.1 us against 15.7, of 262144 49 against
+// 59), so a batch's first move waits for what comes next.
+static int move_engine(rk_batch *b, const rk_batch::Move &m) {
+    hipError_t e = hipMemcpyAsync(m.dst, m.src, (size_t)m.n * 4, m.kind, b->a->d->stream);
+    return e == hipSuccess ? RK_OK : latch(b, hip_fail(b->a->d, e, m.what));
+}
+
+static int move_kernel(rk_batch *b, const rk_batch::Move &m) {
+    ProfScope p(b->a->d, b->a->d->stream, "batch_move");
+    launch_copy(m.src, m.dst, m.n, b->a->d->stream);
+    return launched(b, m.what);
+}
+
+static int move_words(rk_batch *b, const rk_batch::Move &m) {
+    if (m.n <= kBlitWords || m.n > kMoveWords) return move_engine(b, m);
+    if (b->ops > 1) return move_kernel(b, m);
+    b->first = m;
+    return RK_OK;
+}
+
+// The start of each of the batch's operations: the held move goes first.
+static int next_op(rk_batch *b) {
+    if (!b) return RK_ERR_ARGS;
+    if (b->err) return b->err;
+    b->ops++;
+    if (b->first.n == 0) return RK_OK;
+    const rk_batch::Move m = b->first;
+    b->first.n = 0;
+    return move_kernel(b, m);
 }
 
 }  // namespace rk
@@ -241,8 +273,7 @@ int rk_batch_begin(rk_arena *a, rk_batch **out) {
 }
 
 int rk_batch_write(rk_batch *b, int64_t off, const float *data, int64_t n) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     if (n == 0) return RK_OK;
     if (!data) return latch(b, fail(b->a->d, RK_ERR_ARGS, "rk_batch_write: null data"));
     rk_arena *a = b->a;
@@ -253,12 +284,11 @@ int rk_batch_write(rk_batch *b, int64_t off, const float *data, int64_t n) {
     float *st = a->staging + b->staged;
     memcpy(st, data, (size_t)n * 4);
     b->staged += n;
-    return move_words(b, dst, a->staging_d + (st - a->staging), n, hipMemcpyHostToDevice, "batch write");
+    return move_words(b, {dst, a->staging_d + (st - a->staging), n, hipMemcpyHostToDevice, "batch write"});
 }
 
 int rk_batch_read(rk_batch *b, int64_t off, float *dst, int64_t n) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     if (n == 0) return RK_OK;
     if (!dst) return latch(b, fail(b->a->d, RK_ERR_ARGS, "rk_batch_read: null destination"));
     rk_arena *a = b->a;
@@ -266,7 +296,7 @@ int rk_batch_read(rk_batch *b, int64_t off, float *dst, int64_t n) {
         return latch(b, fail(a->d, RK_ERR_ARGS, "gpu: batch moves more than its staging holds"));
     const float *src = span(b, off, n, "read");
     if (!src) return b->err;
-    if (int rc = move_words(b, a->staging_d + b->staged, src, n, hipMemcpyDeviceToHost, "batch read")) return rc;
+    if (int rc = move_words(b, {a->staging_d + b->staged, src, n, hipMemcpyDeviceToHost, "batch read"})) return rc;
     b->reads.push_back({dst, b->staged, n});
     b->staged += n;
     return RK_OK;
@@ -275,8 +305,7 @@ int rk_batch_read(rk_batch *b, int64_t off, float *dst, int64_t n) {
 // internal/gpu/batch.go:212-269 MatVecs: the input quantized once into the
 // arena's scratch, each matrix's rows to its own offset.
 int rk_batch_matvecs(rk_batch *b, int32_t n, rk_matrix *const *ms, const int64_t *out_offs, int64_t in_off) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     if (n <= 0) return RK_OK;
     rk_arena *a = b->a;
     rk_device *d = a->d;
@@ -309,8 +338,7 @@ int rk_batch_matvecs(rk_batch *b, int32_t n, rk_matrix *const *ms, const int64_t
 // codes four a word (little-endian, code j in byte j) at qx_off and its
 // block scales at xs_off (internal/gpu/kernels.go:323-353).
 int rk_batch_quantize(rk_batch *b, int64_t in, int64_t n) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     rk_arena *a = b->a;
     if (a->qx_off < 0) return latch(b, fail(a->d, RK_ERR_ARGS, "gpu: arena has no scratch for quantized inputs"));
     if (n % 32 != 0 || n > kMaxCols) return latch(b, fail(a->d, RK_ERR_ARGS, "gpu: quantize of %lld floats", (long long)n));
@@ -336,8 +364,7 @@ int rk_batch_quantize(rk_batch *b, int64_t in, int64_t n) {
 // an input block holding an infinity or NaN, reads as NaN, the CPU path's
 // value in num.ActFP8.Vals; the reference's Vulkan kernel gives ±480 there.)
 int rk_batch_quantize_fp8(rk_batch *b, int64_t in, int64_t n) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     rk_arena *a = b->a;
     if (a->qx_off < 0) return latch(b, fail(a->d, RK_ERR_ARGS, "gpu: arena has no scratch for quantized inputs"));
     if (n % 32 != 0 || n > kMaxCols) return latch(b, fail(a->d, RK_ERR_ARGS, "gpu: quantize of %lld floats", (long long)n));
@@ -365,8 +392,7 @@ int rk_batch_quantize_fp8(rk_batch *b, int64_t in, int64_t n) {
 // quantized into the scratch first (input k at k·cols codes).
 int rk_batch_expert_matvecs(rk_batch *b, rk_matrix *m, int64_t per_expert, int64_t ids, int32_t slots, int64_t in,
                             int64_t in_stride, int32_t div, int64_t out, int64_t out_stride) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     rk_arena *a = b->a;
     rk_device *d = a->d;
     if (!m || m->d != d || m->kind != RK_FP4 || per_expert <= 0 || m->rows % per_expert != 0)
@@ -417,8 +443,7 @@ int rk_batch_expert_matvecs(rk_batch *b, rk_matrix *m, int64_t per_expert, int64
 // 5120x8192), so the weights are read once an input.
 int rk_batch_matvecs_batch(rk_batch *b, rk_matrix *m, int64_t out, int64_t out_stride, int64_t in, int64_t in_stride,
                            int32_t n) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     if (!m || m->d != b->a->d) return latch(b, fail(b->a->d, RK_ERR_ARGS, "gpu: matrix on another device"));
     for (int32_t j = 0; j < n; j++) {
         const int64_t o = out + j * out_stride;
@@ -430,8 +455,7 @@ int rk_batch_matvecs_batch(rk_batch *b, rk_matrix *m, int64_t out, int64_t out_s
 
 // internal/gpu/dsbatch.go:60-74 ActQuantInPlace and FP4QuantInPlace.
 int rk_batch_act_quant_inplace(rk_batch *b, int64_t off, int64_t n) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     if (n < 0 || n % 32 != 0) return latch(b, fail(b->a->d, RK_ERR_ARGS, "gpu: act quant of %lld floats", (long long)n));
     float *x = span(b, off, n, "act quant");
     if (!x) return b->err;
@@ -441,8 +465,7 @@ int rk_batch_act_quant_inplace(rk_batch *b, int64_t off, int64_t n) {
 }
 
 int rk_batch_fp4_quant_inplace(rk_batch *b, int64_t off, int64_t n, int32_t e4m3) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     if (n < 0 || n % (e4m3 ? 16 : 32) != 0)
         return latch(b, fail(b->a->d, RK_ERR_ARGS, "gpu: fp4 quant of %lld floats", (long long)n));
     float *x = span(b, off, n, "fp4 quant");
@@ -455,8 +478,7 @@ int rk_batch_fp4_quant_inplace(rk_batch *b, int64_t off, int64_t n, int32_t e4m3
 // internal/gpu/batch.go:282-287 RMSNorm.
 int rk_batch_rmsnorm(rk_batch *b, rk_vectors *vecs, int64_t in, int64_t out, int64_t w, int32_t n, int32_t segs,
                      int64_t stride, float recip_n, float eps) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     if (n <= 0 || segs <= 0 || (segs > 1 && stride < 0))
         return latch(b, fail(b->a->d, RK_ERR_ARGS, "rk_batch_rmsnorm: bad shape"));
     const int64_t extent = (int64_t)(segs - 1) * stride + n;
@@ -471,8 +493,7 @@ int rk_batch_rmsnorm(rk_batch *b, rk_vectors *vecs, int64_t in, int64_t out, int
 
 // internal/gpu/batch.go:289-292 AddVec.
 int rk_batch_addvec(rk_batch *b, rk_vectors *vecs, int64_t out, int64_t v, int64_t n) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     float *o = span(b, out, n, "addvec output");
     const float *vv = o ? vspan(b, vecs, v, n, "addvec vector") : nullptr;
     if (!vv) return b->err;
@@ -484,8 +505,7 @@ int rk_batch_addvec(rk_batch *b, rk_vectors *vecs, int64_t out, int64_t v, int64
 // internal/gpu/batch.go:294-298 Rope.
 int rk_batch_rope(rk_batch *b, int64_t q, int64_t k, int32_t q_dim, int32_t kv_dim, int32_t head_size, int64_t cos,
                   int64_t sin) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     if (head_size <= 0 || head_size % 2 || q_dim % 2 || kv_dim < 0 || kv_dim > q_dim)
         return latch(b, fail(b->a->d, RK_ERR_ARGS, "rk_batch_rope: bad shape"));
     float *qq = span(b, q, q_dim, "rope q");
@@ -500,8 +520,7 @@ int rk_batch_rope(rk_batch *b, int64_t q, int64_t k, int32_t q_dim, int32_t kv_d
 
 // internal/gpu/batch.go:300-303 Copy.
 int rk_batch_copy(rk_batch *b, int64_t src, int64_t dst, int64_t n) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     const float *s = span(b, src, n, "copy source");
     float *t = s ? span(b, dst, n, "copy destination") : nullptr;
     if (!t) return b->err;
@@ -514,8 +533,7 @@ int rk_batch_copy(rk_batch *b, int64_t src, int64_t dst, int64_t n) {
 int rk_batch_attention(rk_batch *b, int64_t q, int64_t keys, int64_t vals, int64_t att, int64_t att_stride, int64_t out,
                        int32_t positions, int32_t heads, int32_t kv_heads, int32_t head_size, int32_t kv_dim,
                        float inv_sqrt) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     if (positions <= 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || head_size <= 0 ||
         (int64_t)kv_heads * head_size > kv_dim || att_stride < positions)
         return latch(b, fail(b->a->d, RK_ERR_ARGS, "rk_batch_attention: bad shape"));
@@ -534,8 +552,7 @@ int rk_batch_attention(rk_batch *b, int64_t q, int64_t keys, int64_t vals, int64
 
 // internal/gpu/batch.go:318-326 Residual.
 int rk_batch_residual(rk_batch *b, int64_t x, int64_t y, int64_t n, int32_t canonical) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     float *xx = span(b, x, n, "residual x");
     const float *yy = xx ? span(b, y, n, "residual y") : nullptr;
     if (!yy) return b->err;
@@ -546,8 +563,7 @@ int rk_batch_residual(rk_batch *b, int64_t x, int64_t y, int64_t n, int32_t cano
 
 // internal/gpu/batch.go:328-331 SiluMul.
 int rk_batch_silumul(rk_batch *b, int64_t a_off, int64_t b_off, int64_t n) {
-    if (!b) return RK_ERR_ARGS;
-    if (b->err) return b->err;
+    if (int rc = next_op(b)) return rc;
     float *aa = span(b, a_off, n, "silumul a");
     const float *bb = aa ? span(b, b_off, n, "silumul b") : nullptr;
     if (!bb) return b->err;
@@ -561,6 +577,7 @@ int rk_batch_submit(rk_batch *b) {
     if (!b) return RK_ERR_ARGS;
     rk_arena *a = b->a;
     rk_device *d = a->d;
+    if (b->err == RK_OK && b->first.n) (void)move_engine(b, b->first);  // the batch's only operation
     int rc = b->err;
     hipError_t e = hipStreamSynchronize(d->stream);
     if (e != hipSuccess) {
