@@ -13,6 +13,7 @@
 // The widest input and output of one product (internal/gpu/device.go:197-200).
 constexpr int64_t kMaxCols = (int64_t)1 << 18;
 constexpr int64_t kMaxRows = (int64_t)1 << 20;
+constexpr int64_t kOutWords = (int64_t)1 << 16;
 
 namespace rk {
 // Ownership of a device across calls: a batch holds it from begin to submit
@@ -76,6 +77,7 @@ struct rk_device {
     int8_t *qx = nullptr;
     float *xs = nullptr;
     int32_t *xsum = nullptr;
+    float *out = nullptr;  // kOutWords: outputs of calls of many launches, copied together
     float *h_stage = nullptr, *h_stage_d = nullptr;  // the same words, as the host and as kernels address them
     // Scratch of the batched products (rk_matmul_t*), grown on demand:
     // quantized inputs [tokens][cols] (codes; scales and code sums per block),

@@ -634,3 +634,28 @@ def test_output_over_the_input(dev):
         arena.free()
         for m in ms:
             m.free()
+
+
+@pytest.mark.parametrize("rows", [100, 14000])
+def test_host_products_of_many_matrices(dev, rows):
+    """Six block-scaled matrices of one host call: their outputs copied over
+    together, and (past 65536 rows in all) stored by the products."""
+    rng = np.random.default_rng(rows)
+    cols = 64
+    x = mx_input(rng, cols, specials=True)
+    ms, want = [], []
+    for i in range(6):
+        n = rows + 3 * i
+        if i % 2:
+            w, s = rng.integers(0, 256, n * cols // 2).astype(np.uint8), random_scales(rng, n * cols // 32)
+            want.append(oracle.matvec_fp4(w, s, x, n, cols))
+        else:
+            w, s = random_fp8(rng, n, cols)
+            want.append(oracle.matvec_fp8(w, s, x, n, cols))
+        ms.append(dev.upload_mx(rkhip.FP4 if i % 2 else rkhip.FP8, n, cols, w, s))
+    try:
+        for got, w in zip(dev.matvecs(ms, x), want):
+            same_bits(got, w, f"{w.size} rows")
+    finally:
+        for m in ms:
+            m.free()
