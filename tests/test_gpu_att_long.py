@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 
 from oracle.model import Config, Stage
-from test_gpu_fused_stage import coded_model, make_stage, same_bits
+from test_gpu_fused_stage import coded_model, make_stage, oracle_generate, same_bits
+from test_gpu_stage_seqs import seqs_generate
 
 pytestmark = pytest.mark.gpu
 
@@ -47,4 +48,52 @@ def test_long_context_rows(dev, heads, kv_heads, hd, scale):
             st.free()
             for mt in mats:
                 mt.free()
+    assert dev.used == 0
+
+
+# (a context of 4100: a prompt's values past 1024 positions by the kernel of
+# the decode steps, else by two workgroups a CU)
+@pytest.mark.parametrize("heads,kv_heads,hd,ctx", [(4, 2, 128, 1200), (4, 2, 128, 4100), (4, 1, 64, 1200)])
+def test_infinity_and_nan_rows(dev, heads, kv_heads, hd, ctx):
+    """A position whose activations hold an infinity (its key and value are
+    NaNs): the positions before it are untouched, those after it as the
+    oracle's, in a prompt and in decode steps."""
+    c = Config(dim=96, hidden=64, layers=1, heads=heads, kv_heads=kv_heads, head_dim=hd, vocab=50, seq_len=ctx,
+               dtype="q8_0")
+    m = coded_model(c, 21, 1e-3, 1e-2)
+    rng = np.random.default_rng(5)
+    xs = rng.normal(0, 1, (1110, c.dim)).astype(np.float32)
+    xs[1100, 7] = np.inf
+    cpu = Stage(m, 1200)
+    want = np.stack([cpu.forward(x.copy(), t) for t, x in enumerate(xs)])
+    st, mats = make_stage(dev, m, ctx)
+    try:
+        got = np.concatenate([st.forward(xs[:1105], 0)] + [st.forward(xs[t], t) for t in range(1105, 1110)])
+        for t in range(1110):
+            same_bits(got[t], want[t], f"position {t}")
+    finally:
+        st.free()
+        for mt in mats:
+            mt.free()
+    assert dev.used == 0
+
+
+@pytest.mark.parametrize("lens", [(1100, 3, 1, 40), (1022, 3, 1, 40)])
+@pytest.mark.parametrize("heads,kv_heads,hd", [(4, 2, 128), (4, 2, 64)])
+def test_sequences_of_a_long_context(dev, lens, heads, kv_heads, hd):
+    """Sequences side by side in a context of 1300: each one's position and
+    caches, a prompt past 1024 positions (no batches shared), and one whose
+    steps cross them."""
+    c = Config(dim=96, hidden=64, layers=1, heads=heads, kv_heads=kv_heads, head_dim=hd, vocab=50, seq_len=1300,
+               dtype="q8_0")
+    m = coded_model(c, 22, 1e-3, 1e-2)
+    rng = np.random.default_rng(6)
+    prompts = [[int(t) for t in rng.integers(0, c.vocab, n)] for n in lens]
+    steps = 6
+    lg, toks = seqs_generate(dev, m, prompts, steps, 1300)
+    for z, p in enumerate(prompts):
+        want_t, want_l = oracle_generate(m, p, steps, 1300)
+        for k in range(steps):
+            same_bits(lg[k, z], want_l[k], f"sequence {z} (prompt {len(p)}), step {k}")
+        assert toks[z] == want_t, f"sequence {z} tokens"
     assert dev.used == 0

@@ -106,8 +106,8 @@ def test_argument_errors(dev):
 
 # Sizes about the tiles' edges (32 outputs a side in f32; 128, 64 and 32 in
 # i8, by the number of tiles), the staged slices' (64 positions; 128, 256 and
-# 512) and the loads' (4 floats, 16 bytes), on host buffers and on device
-# pointers off their alignment.
+# 512) and the loads' (4 floats, 16 bytes); int8 on device pointers off their
+# alignment too.
 TILE_SHAPES = [(32, 64, 32), (33, 65, 31), (31, 63, 97), (1, 1, 1), (2, 15, 3), (64, 128, 260), (513, 17, 65),
                (300, 130, 70)]
 
@@ -175,3 +175,59 @@ def test_f32_more_tiles_than_a_grid_dimension(dev):
             assert np.array_equal(bits(np.asarray(g)), bits(np.float32(0) + a[i] * b)), i
     finally:
         arena.free()
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 65, 31), (64, 128, 260), (2, 15, 3), (40, 200, 70)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_f32_infinities_and_nans(dev, m, k, n, off):
+    """The matrix core's products of infinities, NaNs of any payload and
+    zeros of both signs, and their sums, on device pointers at and off their
+    16-byte alignment."""
+    rng = np.random.default_rng(m + 31 * k + 7 * n)
+    odd = np.array([0x7F800000, 0xFF800000, 0x7FA00001, 0xFFC12345, 0x80000000, 0, 0x7F7FFFFF, 1], np.uint32).view(np.float32)
+
+    def draw(rows, cols):
+        v = awkward(rng, rows * cols, 1.0)
+        hit = rng.random(v.size) < 2.0 / k  # most rows and columns hold one or two
+        v[hit] = rng.choice(odd, hit.sum())
+        return v.reshape(rows, cols)
+
+    a, b = draw(m, k), draw(k, n)
+    want = bits(oracle.tensor_matmul_f32(a, b, False))
+    at_a, at_b = off, (m * k + 3 & ~3) + off
+    at_c = at_b + k * n
+    arena = dev.arena(at_c + m * n, at_c + 2 * m * n)
+    try:
+        for transposed, y in ((0, b), (1, np.ascontiguousarray(b.T))):
+            q = arena.begin()
+            q.write(at_a, a.ravel())
+            q.write(at_b, y.ravel())
+            q.submit()
+            dev._check(rkhip.lib().rk_tensor_matmul_device(dev.h, rkhip.TENSOR_F32, transposed, m, k, n,
+                                                           arena.device_ptr(at_a), arena.device_ptr(at_b),
+                                                           arena.device_ptr(at_c), None))
+            q = arena.begin()
+            got = q.read(at_c, m * n)
+            q.submit()
+            assert np.array_equal(bits(np.asarray(got)).reshape(m, n), want)
+    finally:
+        arena.free()
+
+
+# More than 65536 positions (the matrix core's sums start again and are added
+# with wraparound) in the 64 x 64 and the 128 x 64 tiles. a_ip = u_i s_p and
+# b_pj = v_j t_p, so c_ij = u_i v_j sum(s_p t_p).
+@pytest.mark.parametrize("m,n", [(768, 704), (2048, 1024)])
+def test_i8_restarts_in_the_wide_tiles(dev, m, n):
+    rng = np.random.default_rng(m)
+    k = 131072 + 100
+    u, v = rng.integers(-127, 128, m), rng.integers(-127, 128, n)
+    s = np.ones(k, np.int8)
+    t = np.ones(k, np.int8)
+    t[rng.integers(0, k, 1000)] = -1  # 127 * 127 * 129000 leaves int32's range
+    u[:3], v[:2] = 127, (127, -127)
+    want = (np.outer(u, v).astype(np.int64) * int(t.astype(np.int64).sum())).astype(np.uint32).view(np.int32)
+    a = u.astype(np.int8)[:, None] * s
+    b = t[:, None] * v.astype(np.int8)
+    assert np.array_equal(dev.tensor_matmul(a, b), want)
+    assert np.array_equal(dev.tensor_matmul(a, np.ascontiguousarray(b.T), transposed=True), want)
