@@ -49,12 +49,13 @@ __global__ __launch_bounds__(256) void att_scores_long_kernel(const float *q, co
                                                               int kv_heads, int kv_mul, int split, int kv_dim,
                                                               float inv_sqrt) {
     __shared__ __align__(16) float sq[kLongMaxMul * kLongHs];
-    const int z = blockIdx.z;
+    const int tokens = (int)gridDim.z / split, z = (int)blockIdx.z % tokens;
     const int T = att_position(ctl, bt, z) + 1;
     const int t0 = blockIdx.y * kLongTile;
     if (t0 >= T) return;
-    const int g = (int)blockIdx.x / split, part_of = (int)blockIdx.x % split;
-    const int whole = kv_heads * ((T + kLongTile - 1) / kLongTile) * (int)gridDim.z;  // one a kv head and tile
+    // the shares lie in z, so that the first ones alone go round the XCDs
+    const int g = blockIdx.x, part_of = (int)blockIdx.z / tokens;
+    const int whole = kv_heads * ((T + kLongTile - 1) / kLongTile) * tokens;  // one a kv head and tile
     const int parts = min(split, max(1, kLongWgs / whole));
     const int share = (kv_mul + parts - 1) / parts;
     const int m0 = part_of * share, m1 = min(kv_mul, m0 + share);  // its heads
@@ -284,7 +285,7 @@ bool launch_att_scores_long(const float *q, const float *keys, float *att, int32
     // (where the device holds the positions, there may be one tile a token)
     const int whole = kv_heads * tokens * (ctl || bt.pos ? 1 : tiles);
     const int split = std::min(std::min(kv_mul, kLongSplit), std::max(1, kLongWgs / whole));
-    const dim3 grid(kv_heads * split, tiles, tokens);
+    const dim3 grid(kv_heads, tiles, tokens * split);
     RK_LAUNCH(att_scores_long_kernel, grid, dim3(256), 0, s, q, keys, att, att_stride, ctl, bt, kv_heads, kv_mul, split,
               kv_dim, inv_sqrt);
     return true;
