@@ -29,7 +29,7 @@ namespace {
 constexpr int kLongHs = 128;       // head size of the scores kernel
 constexpr int kLongTile = 64;      // positions a scores workgroup
 constexpr int kLongMaxMul = 16;    // query heads a kv head
-constexpr int kLongSplit = 4;      // scores workgroups a kv head and tile, at most
+constexpr int kLongSplitLog2 = 2;  // four scores workgroups a kv head and tile, or one
 constexpr int kLongWgs = 512;      // scores workgroups that keep the chip busy
 constexpr int kLongThreads = 512;  // values: waves 0-3 (0 adds), waves 4-7 load and multiply
 constexpr int kLongWaves = kLongThreads / 64;
@@ -42,24 +42,30 @@ constexpr int kLongChunk = 256;    // positions a product tile
 // thread (position tid/4, part tid%4) keeps its key's elements 8·part .. +7 of
 // each 32-element step in registers and runs the heads over them, as
 // quad_dot32 (the running sums j = 8·part .. +7, combined by DPP). A kv head's
-// `split` workgroups share its query heads while the positions so far leave
+// 2^split_log2 workgroups share its query heads while the positions so far leave
 // workgroups of the chip idle; from there on the first takes them all.
 __global__ __launch_bounds__(256) void att_scores_long_kernel(const float *q, const float *keys, float *att,
                                                               int32_t att_stride, const int32_t *ctl, AttBatch bt,
-                                                              int kv_heads, int kv_mul, int split, int kv_dim,
+                                                              int kv_heads, int kv_mul, int split_log2, int kv_dim,
                                                               float inv_sqrt) {
     __shared__ __align__(16) float sq[kLongMaxMul * kLongHs];
-    const int tokens = (int)gridDim.z / split, z = (int)blockIdx.z % tokens;
+    const int z = (int)blockIdx.z >> split_log2;
     const int T = att_position(ctl, bt, z) + 1;
     const int t0 = blockIdx.y * kLongTile;
     if (t0 >= T) return;
-    // the shares lie in z, so that the first ones alone go round the XCDs
-    const int g = blockIdx.x, part_of = (int)blockIdx.z / tokens;
-    const int whole = kv_heads * ((T + kLongTile - 1) / kLongTile) * tokens;  // one a kv head and tile
-    const int parts = min(split, max(1, kLongWgs / whole));
-    const int share = (kv_mul + parts - 1) / parts;
-    const int m0 = part_of * share, m1 = min(kv_mul, m0 + share);  // its heads
-    if (m0 >= kv_mul) return;
+    const int g = blockIdx.x;
+    int m0 = 0, m1 = kv_mul;  // the workgroup's query heads of the kv head's
+    if (split_log2) {         // uniform (the divisions take 0.5 us)
+        // the shares lie in z, so that the first ones alone go round the XCDs
+        const int split = 1 << split_log2, part_of = (int)blockIdx.z & (split - 1);
+        // workgroups with one a kv head and tile
+        const int whole = kv_heads * ((T + kLongTile - 1) / kLongTile) * ((int)gridDim.z >> split_log2);
+        const int parts = min(split, max(1, kLongWgs / whole));
+        const int share = (kv_mul + parts - 1) / parts;
+        m0 = part_of * share;
+        m1 = min(kv_mul, m0 + share);
+        if (m0 >= kv_mul) return;
+    }
     const int h0 = g * kv_mul;
     const int part = threadIdx.x & 3, t = t0 + (threadIdx.x >> 2);
     const float *kt = keys + att_cache(bt, z) + (int64_t)min(t, T - 1) * kv_dim + (int64_t)g * kLongHs + 8 * part;
@@ -205,51 +211,41 @@ __global__ __launch_bounds__(kLongThreads) void att_values_long_kernel(const flo
             acc = swz_chain_sum(tiles + (c & 1) * (kLongSlice * kLongChunk) + lane * kLongChunk,
                                 min(kLongChunk, T - c * kLongChunk), vr_swz(lane), acc);
     };
-    // While five chunks are left each half loads unconditionally (a test
-    // around a load makes the compiler wait there); the last ones load nothing
+    // Each role has a loop of its own, nch barriers each: with both in one, the
+    // loaded values meet at its joins and are copied there, which waits for
+    // loads just issued. While five chunks are left the loads stand without a
+    // test (it would make the compiler wait too); the last chunks load nothing
     // that nobody reads, for a launch ends when its loads have. (nch >= 5.)
-    int c = 0;
     if (wave >= 4) {
         products(va, 0);
         load(va, 2);
-    }
-    __syncthreads();
-    for (; c + 4 < nch; c += 2) {
-        if (wave == 0) {
-            sums(c);
-        } else if (wave >= 4) {
+        __syncthreads();
+        int c = 0;
+        for (; c + 4 < nch; c += 2) {
             products(vc, c + 1);
+            __builtin_amdgcn_sched_barrier(0);  // the loads into the registers just read, not into others
             load(vc, c + 3);
-        }
-        __syncthreads();
-        if (wave == 0) {
-            sums(c + 1);
-        } else if (wave >= 4) {
+            __syncthreads();
             products(va, c + 2);
+            __builtin_amdgcn_sched_barrier(0);
             load(va, c + 4);
+            __syncthreads();
         }
-        __syncthreads();
-    }
-    const bool four = nch - c > 3;  // three or four chunks: vc holds the second, va the third
-    if (wave == 0) {
-        sums(c);
-    } else if (wave >= 4) {
+        const bool four = nch - c > 3;  // three or four chunks are left
         products(vc, c + 1);
         if (four) load(vc, c + 3);
-    }
-    __syncthreads();
-    if (wave == 0)
-        sums(c + 1);
-    else if (wave >= 4)
-        products(va, c + 2);
-    __syncthreads();
-    if (wave == 0)
-        sums(c + 2);
-    else if (wave >= 4 && four)
-        products(vc, c + 3);
-    if (four) {  // uniform
         __syncthreads();
-        if (wave == 0) sums(c + 3);
+        products(va, c + 2);
+        __syncthreads();
+        if (four) {
+            products(vc, c + 3);
+            __syncthreads();
+        }
+        return;
+    }
+    for (int c = 0; c < nch; c++) {
+        __syncthreads();
+        if (wave == 0) sums(c);
     }
     if (wave != 0) return;
     const int64_t base = (int64_t)z * bt.out_stride + (int64_t)h * hs + e0;
@@ -282,12 +278,15 @@ bool launch_att_scores_long(const float *q, const float *keys, float *att, int32
         return false;
     const int npos = att_positions(ctl, bt, ctx);
     const int tokens = ctl ? 1 : bt.tokens, tiles = (npos + kLongTile - 1) / kLongTile;
-    // (where the device holds the positions, there may be one tile a token)
-    const int whole = kv_heads * tokens * (ctl || bt.pos ? 1 : tiles);
-    const int split = std::min(std::min(kv_mul, kLongSplit), std::max(1, kLongWgs / whole));
-    const dim3 grid(kv_heads, tiles, tokens * split);
-    RK_LAUNCH(att_scores_long_kernel, grid, dim3(256), 0, s, q, keys, att, att_stride, ctl, bt, kv_heads, kv_mul, split,
-              kv_dim, inv_sqrt);
+    // More than four query heads in turn take longer than a launch's start and
+    // end (16 of one kv head, positions up to 4000: 6.5-7.3 us, shared by four
+    // workgroups 3.8-4.1; 7 of one 4.1-4.7 and 3.9-4.1), but workgroups that
+    // exit at once cost too (32768 of them 9 us more than 8192).
+    const int64_t wgs = (int64_t)kv_heads * tokens * tiles;
+    const int split_log2 = kv_mul > 4 && wgs <= 1024 ? kLongSplitLog2 : 0;
+    const dim3 grid(kv_heads, tiles, tokens << split_log2);
+    RK_LAUNCH(att_scores_long_kernel, grid, dim3(256), 0, s, q, keys, att, att_stride, ctl, bt, kv_heads, kv_mul,
+              split_log2, kv_dim, inv_sqrt);
     return true;
 }
 
