@@ -9,7 +9,7 @@
 //    positions' keys in registers: each key row is read once, not once a
 //    query head (6000 positions, 28 heads on 4: 13.4 -> 5.4 us).
 //  * Four waves load the values two chunks ahead and multiply one ahead, one
-//    wave only adds (the sums 25.5 us of a launch; the launch 65.9 -> 55).
+//    wave only adds (the sums 25.5 us of a launch; the launch 65.9 -> 54).
 // Forming the softmax's sum in parallel (exactly: the sum as an integer on
 // its binade's grid, each thread's terms as how far they move an even and an
 // odd one, a scan, again after each thread that leaves the binade) measured

@@ -21,6 +21,7 @@
 // registers, many waves fit a CU, and a part is waited for by count, without
 // a barrier. The input is staged in LDS the same way (kDenseX elements at a
 // time for wider rows). Up to three matrices of one input share a launch.
+// Narrow rows: dense_narrow_kernel.
 //
 // What bounds it: HBM, then the launch and the input's way into LDS for the
 // smaller ones. MI355X, bfloat16 (us, weights past the MALL; before: rows

@@ -172,8 +172,6 @@ bool launch_att_scores_qkn(const float *q_raw, const float *k_raw, const float *
                            float *keys, float *vals, float *att, int32_t att_stride, const int32_t *ctl,
                            const AttBatch &bt, int ctx, int heads, int kv_heads, int hs, int kv_dim, float inv_sqrt,
                            hipStream_t s);
-// Batches up to 1024 positions (head size a multiple of 32) run a group of
-// tokens per workgroup (rk_attn_batch.hip); the results are the same.
 // The scores and the softmax with the weighted values for contexts past
 // kAttLongCtx (rk_attn_long.hip), the same results; false: another shape.
 constexpr int kAttLongCtx = 1024;
@@ -183,6 +181,8 @@ bool launch_att_scores_long(const float *q, const float *keys, float *att, int32
 bool launch_att_values_long(const float *att, int32_t att_stride, const float *vals, float *out, const int32_t *ctl,
                             const AttBatch &bt, int ctx, int heads, int kv_heads, int hs, int kv_dim, int8_t *qx,
                             float *xs, int32_t *xsum, hipStream_t s);
+// Batches up to 1024 positions (head size a multiple of 32) run a group of
+// tokens per workgroup (rk_attn_batch.hip); the results are the same.
 bool att_group_fits(const AttBatch &bt, int hs, int kv_dim);
 void launch_att_scores_group(const float *q, const float *keys, float *att, int32_t att_stride, const AttBatch &bt,
                              int heads, int kv_heads, int kv_dim, float inv_sqrt, hipStream_t s);

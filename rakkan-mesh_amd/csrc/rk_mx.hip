@@ -35,12 +35,11 @@
 // wider than the workgroup's lanes take several chunks, the chain carried
 // across them. With a slot table the grid's second dimension runs selected
 // experts (ExpertMatVecs). A lane quantizes its own input slice while the
-// weights are on their way (mx_quantize): a product takes 1.1-2.3 us longer
-// (32768x1280 E4M3 11.1 -> 13.4, 5120x8192 10.8 -> 12.0, six experts of
-// 2304x5120 E2M1 12.4 -> 13.5, of 5120x2304 11.8 -> 13.6) and the launch
-// before it, 3.4 us and a gap an input, goes (those two projections and three
-// expert products, ten quantized inputs: 143.6 -> 125.5 us). Also here: the in-place E4M3 / E2M1 quantizers
-// of the DeepSeek batch (ActQuantInPlace, FP4QuantInPlace).
+// weights are on their way (mx_quantize), where that takes less than a launch
+// before the product (mx_floats_pay): two E4M3 projections and three products
+// of six E2M1 experts, ten quantized inputs, 143.6 -> 125.5 us. Also here: the
+// in-place E4M3 / E2M1 quantizers of the DeepSeek batch (ActQuantInPlace,
+// FP4QuantInPlace).
 #include <algorithm>
 #include <mutex>
 
@@ -556,8 +555,8 @@ struct MxTune {
     int nb, g, waves;
 };
 constexpr MxTune kMxTune[] = {
-    {true, 160, 1, 3},  // 5120 columns: 13824x5120 11.8 us against 14.3 (G = 2, 5 waves)
-    {true, 72, 3, 4},   // 2304 columns: 5120x2304 5.4 us against 6.4 (G = 7, 8 waves)
+    {true, 160, 1, 3},  // 5120 columns: 13824x5120 11.8 us against 16.0 (G = 2, 5 waves), six experts of 2304 12.3, 16.6
+    {true, 72, 3, 4},   // 2304 columns: 5120x2304 5.6 us against 7.0 (G = 7, 8 waves), six experts of 5120 12.8, 13.7
 };
 
 MxShape mx_shape(bool fp4, int nb) {

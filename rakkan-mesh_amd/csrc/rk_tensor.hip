@@ -11,9 +11,10 @@
 // vector ALU does the adds alone, in order. What bounds it: an add and a
 // product a position, 16 adds (2.3 cycles each) and one matrix instruction
 // (34 cycles) per 1024 products, which measured one after the other on
-// MI355X, not together: 24.5 us of a 1024 x 784 x 1024 product. It takes 38
-// us (75 us with two outputs a side a thread from LDS, products on the vector
-// ALU: operand reads, tests and the loads' latency).
+// MI355X, not together: 24.5 us of a 1024 x 784 x 1024 product. It takes 35-36
+// us (two outputs a side a thread from LDS, products on the vector ALU: 64,
+// and 82 with inputs not in the caches): operand reads, tests and the loads'
+// latency are the rest.
 //
 // i8 (tensor.go:328-335): c_ij = Σ int32(a_ip)·int32(b_pj) with Go's int32
 // wraparound. Integer sums are exact in any order, so the sums run on int8
@@ -22,9 +23,9 @@
 // matrix core) and the partials are added with wrapping integer adds. What
 // bounds it: LDS reads and the staging of slices (16 bytes a lane and row;
 // b[k][n] turned in registers, 4x4 bytes at a time, so that both operands
-// read 16 positions of a row or column as one LDS load). 2048^3: 25.5 us,
-// 337 TMAC/s (21 us with b[n][k]), against 226 us with byte loads, 8-byte
-// LDS reads and no load in flight during the sums.
+// read 16 positions of a row or column as one LDS load). 2048^3: 22-23 us, 380
+// TMAC/s (20 us with b[n][k]), against 221 us with byte loads, 8-byte LDS
+// reads and no load in flight during the sums.
 //
 // Both load the next slice while this one is summed (two LDS slices, one
 // barrier a slice). A slice that is whole takes no tests: a test around a
@@ -444,9 +445,9 @@ static void launch_tensor_i8(const int8_t *a, const int8_t *b, int32_t *c, int64
     // The largest tile that still gives the chip's 256 CUs a workgroup or two
     // each; below 128 tiles of 64 the 32 x 32 one, whose four waves share a
     // slice of 512 positions, unless k would leave most of that slice empty.
-    // Measured (us, k x n operand b): 2048^3 25.5 / 33.5 at 64 / 105 at 32;
-    // 1024^3 9.7 / 7.4 / 16.4; 256 x 2048 x 256 15.2 / 11.1 / 6.4;
-    // 118 x 45 x 279 6.3 / 4.9 / 6.2.
+    // Measured (us, k x n operand b; 128 x 64, 64 x 64, 32 x 32): 2048^3 22.8,
+    // 33.5, 105; 1024^3 9.7, 7.4, 16.4; 256 x 2048 x 256 15.2, 11.1, 6.4;
+    // 118 x 45 x 279 6.3, 4.9, 6.2.
     if (tiles_of(m, n, 128, 64) >= 256)
         launch_tensor_i8_t<128, 64, 128, 2, 2, 1, TRANS>(a, b, c, m, k, n, s);
     else if (tiles_of(m, n, 64, 64) >= 128 || k < 512)
