@@ -178,9 +178,6 @@ constexpr int kAttLongCtx = 1024;
 bool launch_att_scores_long(const float *q, const float *keys, float *att, int32_t att_stride, const int32_t *ctl,
                             const AttBatch &bt, int ctx, int heads, int kv_heads, int hs, int kv_dim, float inv_sqrt,
                             hipStream_t s);
-bool launch_att_values_long(const float *att, int32_t att_stride, const float *vals, float *out, const int32_t *ctl,
-                            const AttBatch &bt, int ctx, int heads, int kv_heads, int hs, int kv_dim, int8_t *qx,
-                            float *xs, int32_t *xsum, hipStream_t s);
 // Batches up to 1024 positions (head size a multiple of 32) run a group of
 // tokens per workgroup (rk_attn_batch.hip); the results are the same.
 bool att_group_fits(const AttBatch &bt, int hs, int kv_dim);

@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <mutex>
 
+#include "rk_attn_long.h"
 #include "rk_attn_reg.h"
 #include "rk_dev.h"
 #include "rk_fused.h"
@@ -1144,6 +1145,50 @@ constexpr size_t kValMaxDynLds = kMaxLdsBytes - 1024;
 
 int att_values_max_ctx() { return (int)(kValMaxDynLds / 4 - 2 * kValSlice * val_pitch(kValChunk)) & ~3; }
 
+// The values in a context past kVrMaxCtx positions, by the position: later
+// ones by rk_attn_long.h, earlier ones from registers or, with more workgroups
+// than CUs (many), by four waves in chunks, which load while they sum (a
+// position of 8192, us: 50, a decode step, long 7.0, registers 5.2, chunks
+// 4.7; 1000, 16 sequences of 32 heads of 64, registers 55.5, chunks 48.6).
+__global__ __launch_bounds__(kLongThreads) void att_values_long_kernel(const float *att, int32_t att_stride,
+                                                                       const float *vals, float *out,
+                                                                       const int32_t *ctl, AttBatch bt, int kv_mul,
+                                                                       int hs, int kv_dim, int nsl, int ctx_pad,
+                                                                       int8_t *qx, float *xs, int32_t *xsum,
+                                                                       int many) {
+    const int z = blockIdx.y;
+    if (att_position(ctl, bt, z) + 1 > kVrMaxCtx) {  // uniform, as below
+        att_values_long_body(att, att_stride, vals, out, ctl, bt, kv_mul, hs, kv_dim, nsl, ctx_pad, qx, xs, xsum);
+    } else if (many) {
+        if (threadIdx.x >= kValThreads) return;  // whole waves: the barriers count those left
+        att_values_body<true, kValChunk, false>(att, att_stride, vals, out, ctl, bt, kv_mul, hs, kv_dim, ctx_pad, qx,
+                                                xs, xsum, blockIdx.x / nsl, blockIdx.x % nsl, z, nullptr, 0);
+    } else {
+        att_values_reg_body<false>(att, att_stride, vals, out, ctl, bt, kv_mul, hs, kv_dim, nsl, ctx_pad, qx, xs, xsum,
+                                   blockIdx.x, z, nullptr, 0);
+    }
+}
+
+static bool launch_att_values_long(const float *att, int32_t att_stride, const float *vals, float *out,
+                                   const int32_t *ctl, const AttBatch &bt, int ctx, int heads, int kv_heads, int hs,
+                                   int kv_dim, int8_t *qx, float *xs, int32_t *xsum, bool many, hipStream_t s) {
+    const size_t lds = att_values_lds(ctx, kValChunk);  // (no smaller than the other bodies')
+    static_assert(val_pitch(kValChunk) >= kLongChunk && val_pitch(kValChunk) >= kVrChunk, "one size for the three");
+    if (ctx <= kAttLongCtx || hs % kLongSlice != 0 || kv_dim % 4 != 0 || bt.cache_stride % 4 != 0 ||
+        (reinterpret_cast<uintptr_t>(vals) & 15) != 0 || lds > kMaxLdsBytes - 2048)
+        return false;
+    static std::once_flag once;
+    std::call_once(once, [] {
+        (void)hipFuncSetAttribute((const void *)att_values_long_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)(kMaxLdsBytes - 2048));
+    });
+    const int nsl = hs / kLongSlice;
+    RK_LAUNCH(att_values_long_kernel, dim3(heads * nsl, ctl ? 1 : bt.tokens), dim3(kLongThreads), lds, s, att,
+              att_stride, vals, out, ctl, bt, heads / kv_heads, hs, kv_dim, nsl, (ctx + 3) & ~3, qx, xs, xsum,
+              many ? 1 : 0);
+    return true;
+}
+
 void launch_att_values(const float *att, int32_t att_stride, const float *vals, float *out, const int32_t *ctl,
                        const AttBatch &bt, int ctx, int heads, int kv_heads, int hs, int kv_dim, int8_t *qx,
                        float *xs, int32_t *xsum, hipStream_t s, int cu) {
@@ -1185,15 +1230,15 @@ void launch_att_values(const float *att, int32_t att_stride, const float *vals, 
                   (ctx + 3) & ~3, qx, xs, xsum);
         return;
     }
-    // Past kVrMaxCtx positions a workgroup of rk_attn_long.hip has a CU to
-    // itself; more of them than CUs are faster by att_values_kernel where its
-    // LDS leaves a CU room for two (up to 3.8 k positions; a prompt's tokens
+    // Past kVrMaxCtx positions a workgroup of att_values_long_kernel has a CU
+    // to itself; more of them than CUs are faster by att_values_kernel where
+    // its LDS leaves a CU room for two (up to 3.8 k positions; a prompt's tokens
     // 1024-1535 of 32 heads of 128, two layers: 8.4 ms against 10.6; a context
     // of 8192 11.8 and 10.6).
-    const bool two = (int64_t)grid.x * grid.y * grid.z > (cu > 0 ? cu : 256) &&
-                     att_values_lds(ctx, kValChunk) + 1024 <= kMaxLdsBytes / 2;
-    if (!two &&
-        launch_att_values_long(att, att_stride, vals, out, ctl, bt, ctx, heads, kv_heads, hs, kv_dim, qx, xs, xsum, s))
+    const bool many = (int64_t)grid.x * grid.y * grid.z > (cu > 0 ? cu : 256);
+    const bool two = many && att_values_lds(ctx, kValChunk) + 1024 <= kMaxLdsBytes / 2;
+    if (!two && launch_att_values_long(att, att_stride, vals, out, ctl, bt, ctx, heads, kv_heads, hs, kv_dim, qx, xs,
+                                       xsum, many, s))
         return;
     if (vec)
         RK_LAUNCH((att_values_kernel<true, kValChunk>), grid, dim3(kValThreads), att_values_lds(ctx, kValChunk), s, att,

@@ -78,21 +78,22 @@ def test_infinity_and_nan_rows(dev, heads, kv_heads, hd, ctx):
     assert dev.used == 0
 
 
-@pytest.mark.parametrize("lens", [(1100, 3, 1, 40), (1022, 3, 1, 40)])
-@pytest.mark.parametrize("heads,kv_heads,hd", [(4, 2, 128), (4, 2, 64)])
-def test_sequences_of_a_long_context(dev, lens, heads, kv_heads, hd):
-    """Sequences side by side in a context of 1300: each one's position and
-    caches, a prompt past 1024 positions (no batches shared), and one whose
-    steps cross them."""
-    c = Config(dim=96, hidden=64, layers=1, heads=heads, kv_heads=kv_heads, head_dim=hd, vocab=50, seq_len=1300,
+@pytest.mark.parametrize("heads,kv_heads,hd,ctx,lens", [
+    (4, 2, 128, 1300, (1100, 3, 1, 40)), (4, 2, 128, 1300, (1022, 3, 1, 40)), (4, 2, 64, 1300, (1100, 3, 1, 40)),
+    (4, 2, 64, 1300, (1022, 3, 1, 40)), (8, 2, 128, 4100, (1100, 3, 1, 40, 7, 200, 64, 2, 1022))])
+def test_sequences_of_a_long_context(dev, heads, kv_heads, hd, ctx, lens):
+    """Sequences side by side in a long context: each one's position and
+    caches, a prompt past 1024 positions (no batches shared), one whose steps
+    cross them, and more values workgroups than CUs."""
+    c = Config(dim=96, hidden=64, layers=1, heads=heads, kv_heads=kv_heads, head_dim=hd, vocab=50, seq_len=ctx,
                dtype="q8_0")
     m = coded_model(c, 22, 1e-3, 1e-2)
     rng = np.random.default_rng(6)
     prompts = [[int(t) for t in rng.integers(0, c.vocab, n)] for n in lens]
     steps = 6
-    lg, toks = seqs_generate(dev, m, prompts, steps, 1300)
+    lg, toks = seqs_generate(dev, m, prompts, steps, ctx)
     for z, p in enumerate(prompts):
-        want_t, want_l = oracle_generate(m, p, steps, 1300)
+        want_t, want_l = oracle_generate(m, p, steps, ctx)
         for k in range(steps):
             same_bits(lg[k, z], want_l[k], f"sequence {z} (prompt {len(p)}), step {k}")
         assert toks[z] == want_t, f"sequence {z} tokens"
